@@ -227,6 +227,8 @@ def lib():
     L.agmi_optimizer_step.argtypes = [c_i, c_i, c_i, c_i64, c_p, c_p, c_p, c_p, c_p, p_d, c_p]
     L.agmi_lse_cotangent_fused.restype = c_i
     L.agmi_lse_cotangent_fused.argtypes = [c_i, ctypes.POINTER(AgmiLseCotangent), c_p, c_sz, c_p]
+    L.agmi_lse_rows_fused.restype = c_i
+    L.agmi_lse_rows_fused.argtypes = [c_i, ctypes.POINTER(AgmiLseCotangent), c_p, c_i64, c_p, c_sz, c_p]
     L.agmi_correlate.restype = c_i
     L.agmi_correlate.argtypes = [c_i, ctypes.POINTER(AgmiCorrelation), c_p]
     _LIB = L
@@ -236,7 +238,7 @@ def lib():
 EXPORTS = (
     "agmi_last_error agmi_version agmi_last_kernel agmi_elementwise agmi_program agmi_compare agmi_cast agmi_map_reduce "
     "agmi_map_reduce_workspace_bytes agmi_map_reduce_static agmi_gemm agmi_gemm_fused agmi_fill agmi_take_rows agmi_sort_rows agmi_cumsum agmi_reverse agmi_triangle agmi_scatter_add_rows agmi_optimizer_step "
-    "agmi_correlate agmi_lse_cotangent_fused agmi_concat agmi_probe_arm agmi_probe_elapsed "
+    "agmi_correlate agmi_lse_cotangent_fused agmi_lse_rows_fused agmi_concat agmi_probe_arm agmi_probe_elapsed "
     "agmi_program_specialize agmi_program_specialized agmi_program_source"
 ).split()
 
@@ -674,17 +676,16 @@ def map_reduce_static(op, red, code, shape, reduce_mask, out, ins):
 
 
 _lse_cot = AgmiLseCotangent()
+LSE_ROWS_MAX_VECTORS = 8192  # 16-byte vectors in the longest row that agmi_lse_rows_fused takes
 
 
-def lse_cotangent(code, x, ans, g, row_sums=None, col_factor=None, scaled=None, col_sums=None):
-    """One pass of ``agmi_lse_cotangent_fused`` over the 2-d operand ``x`` (a tensor, or an :class:`Affine` whose array
-    steps are 2-d broadcast views); ``ans`` and ``g`` are (rows, 1) tensors (``g`` may be broadcast).  Outputs are
-    contiguous tensors or None.  Returns False when the layout is outside what the kernel covers."""
+def _fill_lse_cotangent(x, g, row_sums, col_factor, scaled, col_sums):
+    """The descriptor of one pass over the 2-d operand ``x`` (everything but ``ans``); None when its rows are not contiguous."""
     c = _lse_cot
     raw = x.t if type(x) is Affine else x
     c.rows, c.cols = raw.shape
     if raw.stride(1) != 1 and raw.shape[1] > 1:
-        return False
+        return None
     c.x, c.x_row_stride = raw.data_ptr(), raw.stride(0)
     flags, c.scale, c.shift, c.scale_vec, c.shift_vec = 0, 1.0, 0.0, None, None
     if type(x) is Affine:
@@ -702,13 +703,23 @@ def lse_cotangent(code, x, ans, g, row_sums=None, col_factor=None, scaled=None, 
                 c.shift_vec, c.shift_row_stride, c.shift_col_stride = x.shift.data_ptr(), x.shift.stride(0), x.shift.stride(1)
                 flags |= 8
     c.affine = flags
-    c.ans, c.ans_stride = ans.data_ptr(), ans.stride(0)
     c.g, c.g_stride = g.data_ptr(), g.stride(0)
     c.row_sums = row_sums.data_ptr() if row_sums is not None else None
     c.col_factor = col_factor.data_ptr() if col_factor is not None else None
     c.scaled = scaled.data_ptr() if scaled is not None else None
     c.scaled_row_stride = scaled.stride(0) if scaled is not None else 0
     c.col_sums = col_sums.data_ptr() if col_sums is not None else None
+    return c
+
+
+def lse_cotangent(code, x, ans, g, row_sums=None, col_factor=None, scaled=None, col_sums=None):
+    """One pass of ``agmi_lse_cotangent_fused`` over the 2-d operand ``x`` (a tensor, or an :class:`Affine` whose array
+    steps are 2-d broadcast views); ``ans`` and ``g`` are (rows, 1) tensors (``g`` may be broadcast).  Outputs are
+    contiguous tensors or None.  Returns False when the layout is outside what the kernel covers."""
+    c = _fill_lse_cotangent(x, g, row_sums, col_factor, scaled, col_sums)
+    if c is None:
+        return False
+    c.ans, c.ans_stride = ans.data_ptr(), ans.stride(0)
     ev = _TIMER.begin(("lse_cotangent",)) if _TIMER is not None else None
     probe = _LIB.agmi_probe_arm() if ev is not None else None  # (the tile kernel alone; `ev` brackets it and the finishing kernel)
     rc = _LIB.agmi_lse_cotangent_fused(code, ctypes.byref(c), _workspace().data_ptr(), _WORKSPACE_BYTES, _stream())
@@ -717,10 +728,33 @@ def lse_cotangent(code, x, ans, g, row_sums=None, col_factor=None, scaled=None, 
     if rc:
         _check(rc, "agmi_lse_cotangent_fused")
     if ev is not None:
-        outs = tuple(t for t in (row_sums, scaled, col_sums) if t is not None)
-        _TIMER.end(ev, ("lse_cotangent",), (outs, (x, ans, g) + ((col_factor,) if col_factor is not None else ())),
-                   probe=probe if probe is not None and probe >= 0 else None)
+        _end_lse(ev, probe, x, (ans, g), col_factor, row_sums, scaled, col_sums)
     return True
+
+
+def lse_rows(code, x, g, ans=None, row_sums=None, col_factor=None, scaled=None, col_sums=None):
+    """The same results, and ``ans = logsumexp(x, axis=1)`` itself (a (rows, 1) output tensor, or None), in one pass over
+    ``x`` (``agmi_lse_rows_fused``); without ``col_factor`` the scaled copy is the cotangent itself.  Returns False when the
+    layout is outside what the kernel covers."""
+    c = _fill_lse_cotangent(x, g, row_sums, col_factor, scaled, col_sums)
+    if c is None:
+        return False
+    ev = _TIMER.begin(("lse_rows",)) if _TIMER is not None else None
+    probe = _LIB.agmi_probe_arm() if ev is not None else None
+    ans_ptr, ans_stride = (ans.data_ptr(), ans.stride(0)) if ans is not None else (None, 0)
+    rc = _LIB.agmi_lse_rows_fused(code, ctypes.byref(c), ans_ptr, ans_stride, _workspace().data_ptr(), _WORKSPACE_BYTES, _stream())
+    if rc == -2:  # AGMI_ERR_UNSUPPORTED
+        return False
+    if rc:
+        _check(rc, "agmi_lse_rows_fused")
+    if ev is not None:
+        _end_lse(ev, probe, x, (g,), col_factor, ans, row_sums, scaled, col_sums)
+    return True
+
+
+def _end_lse(ev, probe, x, ins, col_factor, *outs):
+    _TIMER.end(ev, ("lse_cotangent",), (tuple(t for t in outs if t is not None), (x,) + ins + ((col_factor,) if col_factor is not None else ())),
+               probe=probe if probe is not None and probe >= 0 else None)
 
 
 def gemm(code, batch, M, N, K, alpha, A, a_rs, a_cs, a_bs, B, b_rs, b_cs, b_bs, beta, C, ldc, c_bs):

@@ -359,6 +359,395 @@ static int launch_lse_cotangent(const agmi_lse_cotangent &c, void *workspace, si
     return 0;
 }
 
+// ---- the whole reduction and its cotangent in one pass ----------------------------------------------------
+//
+// When the logsumexp itself has not run yet (its value is only wanted by the rules, as under `grad`), a row that
+// fits the registers of a few waves is read ONCE: its maximum and sum of exponentials give ans, and the very
+// exponentials, rescaled, are S.  Bound by HBM: mem read once, the scaled copy written once (the two-pass form reads mem
+// twice).  8192 x 4096 float32: 50 + 4 us (5.4 TB/s in the first kernel) against 75 us in three launches (26.6 + 44.2 + 4.0);
+// 3001 x 1999 float64, whose rows are no whole number of vectors: 33 us against 134 us in six launches.
+//
+// A block of 16 waves works on 16 / WR rows at a time, WR waves to a row, J vectors of 16 bytes per lane; one block per CU walks
+// the rows with a stride, so that column sums stay in registers from row to row and only 256 partial rows
+// reach memory.  The next rows' loads are issued before the current ones are worked on (64 KB in flight per CU at 4096
+// float32 columns; latency x bandwidth is about 50 KB).  Per row there is one exchange between waves and one barrier: each wave
+// takes the exponentials against its OWN maximum m_w and publishes (m_w, sum); after the barrier every wave combines
+// the WR pairs to (m, total) and S is its exponentials times g * exp(m_w - m) / total: one exponential per element, the
+// logarithm is only taken for the value of ans.
+//
+// Rows are addressed through buffer descriptors of exactly one row: elements past its end load as zero (and are turned into
+// -inf, which neither maximum nor sum sees) and stores past it are dropped, dword by dword, so any number of columns
+// and any element alignment takes the same path.  Measured at 8192 x 4096 with the finish: 16 waves, 8 to a row, 2 vectors 54 us; 4
+// to a row, 4 vectors 56; blocks of 8 or 4 waves 53-60 and 63; 16 waves to a row 68; streaming or plain accesses alike.  Vectors that run along the columns (the factor of the pending map, an offset, the
+// factor of the scaled copy) are staged in LDS once per block.
+constexpr int kLseRowsMaxBlocks = 256;                // one block per CU: 16 waves of up to 128 VGPRs (8 of 256) fill it
+constexpr size_t kLseRowsMaxLds = 144 * 1024;         // of the CU's 160 KB, beside the static exchange slots
+
+struct LseRowsParams {
+    int64_t rows, cols;
+    const void *x;
+    int64_t x_rs;
+    double scale, shift;
+    int scalar_steps;       // any of scale / shift present
+    const void *scale_vec;  // per row (scale_rs) unless scale_lds
+    int64_t scale_rs;
+    const void *shift_vec;
+    int64_t shift_rs;
+    const void *g;
+    int64_t g_rs;
+    void *ans;  // may be null
+    int64_t ans_rs;
+    void *row_sums;  // may be null
+    void *scaled;    // may be null
+    int64_t scaled_rs;
+    void *col_out;   // [gridDim.x][cols] partial column sums
+    // the column vectors staged in LDS: source (null: ones), in slots of `lds_pitch` elements
+    const void *scale_src, *factor_src, *shift_src;
+    int factor_slot;  // 0: the same vector as slot 0
+    int shift_slot;   // 0: none
+    int n_slots;
+    int lds_pitch;
+};
+
+typedef unsigned lse_v4u __attribute__((ext_vector_type(4)));
+
+// The matrix is read once and the scaled copy is not read back by this pass: streaming accesses (bit 1 of the policy).
+constexpr int kLseRowsLoadPolicy = 2, kLseRowsStorePolicy = 2;
+
+// the larger of two values; a NaN loses against a number (NaNs reach the result through the sum of exponentials)
+__device__ __forceinline__ float larger(float a, float b) { return __builtin_fmaxf(a, b); }
+__device__ __forceinline__ double larger(double a, double b) { return __builtin_fmax(a, b); }
+
+template <typename T, int NW, int WR, int J, bool COLS>
+__global__ __launch_bounds__(NW * 64) void lse_cotangent_tile_rows(const LseRowsParams p) {
+    constexpr int V = 16 / sizeof(T), R = NW / WR, NT = WR * 64;
+    // sixteen waves of eight vectors: neither the next row nor the exponentials fit beside the row and the column sums
+    constexpr bool kLong = NW == 16 && J == 8;
+    // vectors are worked on one after the other where the temporaries of several exponentials at once would spill
+    constexpr bool kFence = kLong || sizeof(T) == 8;
+    typedef T vec_t __attribute__((ext_vector_type(V)));
+    extern __shared__ __attribute__((aligned(16))) unsigned char lse_lds[];
+    T *const held = reinterpret_cast<T *>(lse_lds);
+    __shared__ T pair_m[2][NW], pair_s[2][NW];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int rg = wave / WR, wr = wave % WR, t = wr * 64 + lane;
+    const int cols = static_cast<int>(p.cols);
+    const T kInf = T(__builtin_huge_val());
+
+    const auto stage = [&](int slot, const void *src) __attribute__((always_inline)) {
+        for (int c = tid; c < p.lds_pitch; c += NW * 64)
+            held[slot * p.lds_pitch + c] = (src != nullptr && c < cols) ? static_cast<const T *>(src)[c] : T(1);
+    };
+    stage(0, p.scale_src);
+    if (p.factor_slot > 0) stage(p.factor_slot, p.factor_src);
+    if (p.shift_slot > 0) stage(p.shift_slot, p.shift_src);
+    __syncthreads();
+
+    const T sc = static_cast<T>(p.scale), sh = static_cast<T>(p.shift);
+    const bool full = cols == NT * J * V;
+    vec_t acc[COLS ? J : 1];
+#pragma unroll
+    for (int j = 0; j < (COLS ? J : 1); ++j)
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[j][v] = T(0);
+
+    const unsigned row_bytes = static_cast<unsigned>(cols) * sizeof(T);
+    // what a row needs besides its elements; fetched before them, so that waiting for it leaves them in flight
+    T g_next = T(0), sr_next = T(1), hr_next = T(0);
+    vec_t next[J];
+    const auto load = [&](int64_t r) __attribute__((always_inline)) {
+        const int64_t rr = r < p.rows ? r : p.rows - 1;  // the same for the whole wave
+        g_next = static_cast<const T *>(p.g)[rr * p.g_rs];
+        if (p.scale_vec != nullptr) sr_next = static_cast<const T *>(p.scale_vec)[rr * p.scale_rs];
+        if (p.shift_vec != nullptr) hr_next = static_cast<const T *>(p.shift_vec)[rr * p.shift_rs];
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<T *>(static_cast<const T *>(p.x) + rr * p.x_rs), 0, row_bytes, 0x00020000);
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+            next[j] = __builtin_bit_cast(vec_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (j * NT + t) * 16, 0, kLseRowsLoadPolicy));
+    };
+
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * R;
+    int64_t base = static_cast<int64_t>(blockIdx.x) * R;
+    if (!kLong) load(base + rg);
+    int slot = 0;
+    for (; base < p.rows; base += stride, slot ^= 1) {
+        const int64_t r = base + rg;
+        const bool valid = r < p.rows;  // the same for the whole wave
+        if (kLong) load(r);
+        const T g = g_next, sr = sr_next, hr = hr_next;
+        vec_t a[J];
+#pragma unroll
+        for (int j = 0; j < J; ++j) a[j] = next[j];
+        // where registers are short the staged vectors are read again for every row (an address the compiler cannot
+        // see through keeps it from loading all of them ahead of the loop)
+        int here = t * V;
+        if (kFence) asm volatile("" : "+v"(here));
+        if (!kLong && base + stride < p.rows) load(r + stride);
+
+        const auto mapped = [&](int j) __attribute__((always_inline)) -> vec_t {
+            if (kLong) {  // (formed anew by each of its three users: kept from one to the next it would be spilled)
+#pragma unroll
+                for (int v = 0; v < V; ++v) {
+                    T kept = a[j][v];
+                    asm volatile("" : "+v"(kept));
+                    a[j][v] = kept;
+                }
+                asm volatile("" : "+v"(here));
+            }
+            const vec_t sv = *reinterpret_cast<const vec_t *>(held + here + j * NT * V);
+            vec_t hv;
+            if (p.shift_slot > 0) hv = *reinterpret_cast<const vec_t *>(held + p.shift_slot * p.lds_pitch + here + j * NT * V);
+            else
+#pragma unroll
+                for (int v = 0; v < V; ++v) hv[v] = hr;
+            vec_t x;
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                T u = a[j][v];
+                if (p.scalar_steps) u = u * sc;
+                // (a factor varies along the rows or along the columns; the other is one, which is exact)
+                u = (u * sv[v]) * sr;
+                if (p.scalar_steps) u = u + sh;
+                u = u + hv[v];
+                x[v] = (full || (j * NT + t) * V + v < cols) ? u : -kInf;
+            }
+            return x;
+        };
+        vec_t e[J];
+        T m = -kInf;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            const vec_t x = mapped(j);
+#pragma unroll
+            for (int v = 0; v < V; ++v) m = larger(x[v], m);
+            if (!kLong) e[j] = x;
+            if (kFence) __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int k = 32; k > 0; k >>= 1) m = larger(__shfl_xor(m, k, 64), m);
+        // an infinite maximum is not subtracted: -inf terms give 0, +inf terms inf and NaNs NaN, as they should
+        const T ms = (m == kInf || m == -kInf) ? T(0) : m;
+        T sum = T(0);
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            const vec_t x = !kLong ? e[j] : mapped(j);
+            T part = T(0);
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                const T y = exp_of_nonpositive(x[v] - ms);
+                if (!kLong) e[j][v] = y;
+                part += y;
+            }
+            sum += part;
+            if (kFence) __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int k = 32; k > 0; k >>= 1) sum += __shfl_xor(sum, k, 64);
+        T top = m, total = sum, own = T(1);
+        if (WR > 1) {
+            if (lane == 0) {
+                pair_m[slot][wave] = m;
+                pair_s[slot][wave] = sum;
+            }
+            // (two sets of slots in turn: a wave writes a set again only after the barrier that follows every read of it)
+            __syncthreads();
+            // lane k takes pair k % WR: one exponential for all of them (a float64 exponential is some fifty instructions)
+            const T mk = pair_m[slot][rg * WR + lane % WR], sk = pair_s[slot][rg * WR + lane % WR];
+            top = mk;
+#pragma unroll
+            for (int k = 1; k < WR; k <<= 1) top = larger(__shfl_xor(top, k, 64), top);
+            const T weight = (top == kInf || top == -kInf) ? T(1) : exp_of_nonpositive(mk - top);
+            total = sk * weight;
+#pragma unroll
+            for (int k = 1; k < WR; k <<= 1) total += __shfl_xor(total, k, 64);
+            own = from_lane(weight, wr);
+        }
+        const bool finite = total - total == T(0) && top - top == T(0);  // (the total is at least one then)
+        if (wr == 0 && valid && (p.ans != nullptr || p.row_sums != nullptr)) {
+            // all -inf: -inf; a +inf present: +inf unless there is a NaN too
+            const T ans = finite ? top + m_log(total) : (total == total ? top : total);
+            if (lane == 0) {
+                if (p.ans != nullptr) static_cast<T *>(p.ans)[r * p.ans_rs] = ans;
+                // the exponentials over their own total add up to one; a row whose logsumexp is not finite holds an
+                // exp(inf - inf) or an exp(NaN)
+                if (p.row_sums != nullptr) static_cast<T *>(p.row_sums)[r] = finite ? g : T(__builtin_nan(""));
+            }
+        }
+        const T bad = total == total ? top : total;  // ans, where it is not finite
+        const T gf = m == -kInf ? T(0) : (g * own) / total;
+        const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(
+            static_cast<T *>(p.scaled) + r * p.scaled_rs, 0, (valid && p.scaled != nullptr) ? row_bytes : 0u, 0x00020000);
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            const vec_t fv = *reinterpret_cast<const vec_t *>(held + p.factor_slot * p.lds_pitch + here + j * NT * V);
+            vec_t s, o;
+            if (!kLong && finite) {  // the same for the whole row
+#pragma unroll
+                for (int v = 0; v < V; ++v) s[v] = e[j][v] * gf;
+            } else {
+                const vec_t x = mapped(j);
+#pragma unroll
+                for (int v = 0; v < V; ++v) s[v] = !kLong || !finite ? g * exp_of_nonpositive(x[v] - bad) : exp_of_nonpositive(x[v] - ms) * gf;
+            }
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                o[v] = fv[v] * s[v];
+                if (COLS && valid) acc[j][v] += a[j][v] * s[v];
+            }
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(lse_v4u, o), out, (j * NT + t) * 16, 0, kLseRowsStorePolicy);
+            if (kFence) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+
+    if (COLS) {
+        // the row groups' column sums, added in group order by the first group
+        __syncthreads();  // (the staged vectors are no longer needed: their memory holds the other groups' sums)
+        vec_t *const parked = reinterpret_cast<vec_t *>(lse_lds);
+        for (int k = 1; k < R; ++k) {
+            if (rg == k) {
+#pragma unroll
+                for (int j = 0; j < J; ++j) parked[j * NT + t] = acc[j];
+            }
+            __syncthreads();
+            if (rg == 0) {
+#pragma unroll
+                for (int j = 0; j < J; ++j) acc[j] = acc[j] + parked[j * NT + t];
+            }
+            __syncthreads();
+        }
+        if (rg == 0) {
+            const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(
+                static_cast<T *>(p.col_out) + static_cast<int64_t>(blockIdx.x) * p.cols, 0, row_bytes, 0x00020000);
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(lse_v4u, acc[j]), out, (j * NT + t) * 16, 0, 0);
+        }
+    }
+}
+
+template <typename T, int NW, int WR, int J>
+static int launch_lse_rows_kernel(const LseRowsParams &p, bool cols, int blocks, size_t lds, hipStream_t s) {
+    const void *kernel = cols ? reinterpret_cast<const void *>(lse_cotangent_tile_rows<T, NW, WR, J, true>)
+                              : reinterpret_cast<const void *>(lse_cotangent_tile_rows<T, NW, WR, J, false>);
+    if (lds > 64 * 1024) {  // has to be asked for
+        if (int rc = hip_check(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)),
+                               "lse_rows LDS size"))
+            return rc;
+    }
+    if (cols) hipLaunchKernelGGL((lse_cotangent_tile_rows<T, NW, WR, J, true>), dim3(blocks), dim3(NW * 64), lds, s, p);
+    else hipLaunchKernelGGL((lse_cotangent_tile_rows<T, NW, WR, J, false>), dim3(blocks), dim3(NW * 64), lds, s, p);
+    return hip_check(hipGetLastError(), "lse_rows launch");
+}
+
+template <typename T>
+static int launch_lse_rows(const agmi_lse_cotangent &c, void *ans_out, int64_t ans_stride, void *workspace, size_t workspace_bytes,
+                           hipStream_t s) {
+    constexpr int V = 16 / sizeof(T);
+    const int64_t nv = ceil_div(c.cols, V);
+    // Waves to a row (wr) and vectors to a lane (j), in blocks of nw waves.  Short rows get one or two waves, with little or
+    // no exchange between waves, once there are rows enough to give every CU a full block of them; longer rows the
+    // fewest waves whose registers hold two rows, the exponentials and the column sums (float64 exponentials need twice the
+    // temporaries, so half the vectors); beyond that sixteen waves of eight vectors, without the next row in flight.
+    constexpr bool kWide = sizeof(T) == 8;
+    const bool many = c.rows >= static_cast<int64_t>(kLseRowsMaxBlocks) * 8;
+    int nw = 16, wr, j;
+    if (nv <= 64) wr = 1, j = 1;
+    else if (nv <= 128 && many) wr = 1, j = 2;
+    else if (nv <= 256 && many) wr = 2, j = 2;
+    else if (nv <= 256) wr = 4, j = 1;
+    else if (nv <= 512) wr = 4, j = 2;
+    else if (nv <= 1024) wr = 8, j = 2;
+    else if (nv <= 2048) wr = 16, j = 2;
+    else if (nv <= 4096) nw = kWide ? 8 : 16, wr = kWide ? 8 : 16, j = kWide ? 8 : 4;
+    else wr = 16, j = 8;
+    // Rows of more than 4096 vectors: the pass without the next row in flight takes 68 / 77 us on 500 x 32768 float32 / 500 x
+    // 16384 float64, the reduction and the tile kernel 65 / 70; those take whole vectors only, so what is left here
+    // are other numbers of columns (250 x 26895 float32: 48 us, five separate kernels 93).
+    if (nv > 8192 || (nv > 4096 && c.cols % V == 0)) {
+        set_error("lse_rows: %lld columns do not fit one block's registers", (long long)c.cols);
+        return AGMI_ERR_UNSUPPORTED;
+    }
+    LseRowsParams p = {};
+    p.rows = c.rows; p.cols = c.cols;
+    p.x = c.x; p.x_rs = c.x_row_stride;
+    p.scale = (c.affine & AGMI_AFFINE_SCALE) ? c.scale : 1.0;
+    p.shift = (c.affine & AGMI_AFFINE_SHIFT) ? c.shift : 0.0;
+    p.scalar_steps = (c.affine & (AGMI_AFFINE_SCALE | AGMI_AFFINE_SHIFT)) != 0;
+    p.n_slots = 1;
+    // (the stride of an axis of extent 1 is never used: any value is as good as 0)
+    const int64_t scale_rs = c.rows == 1 ? 0 : c.scale_row_stride, shift_rs = c.rows == 1 ? 0 : c.shift_row_stride;
+    const int64_t scale_cs = c.cols == 1 ? 0 : c.scale_col_stride, shift_cs = c.cols == 1 ? 0 : c.shift_col_stride;
+    if (c.affine & AGMI_AFFINE_SCALE_AUX) {
+        if (!c.scale_vec || (scale_cs != 0 && (scale_cs != 1 || scale_rs != 0))) {
+            set_error("lse_rows: the array factor must vary along rows only or along columns only (unit stride)");
+            return AGMI_ERR_UNSUPPORTED;
+        }
+        if (scale_cs == 1) p.scale_src = c.scale_vec;
+        else p.scale_vec = c.scale_vec, p.scale_rs = scale_rs;
+    }
+    if (c.affine & AGMI_AFFINE_SHIFT_AUX) {
+        if (!c.shift_vec || (shift_cs != 0 && (shift_cs != 1 || shift_rs != 0))) {
+            set_error("lse_rows: the array offset must vary along rows only or along columns only (unit stride)");
+            return AGMI_ERR_UNSUPPORTED;
+        }
+        if (shift_cs == 1) p.shift_src = c.shift_vec, p.shift_slot = p.n_slots++;
+        else p.shift_vec = c.shift_vec, p.shift_rs = shift_rs;
+    }
+    p.g = c.g; p.g_rs = c.g_stride;
+    p.ans = ans_out; p.ans_rs = ans_stride;
+    p.row_sums = c.row_sums;
+    p.scaled = c.scaled; p.scaled_rs = c.scaled_row_stride;
+    if (c.scaled && c.scaled_row_stride < c.cols) {
+        set_error("lse_rows: the scaled copy needs a row stride >= cols");
+        return AGMI_ERR_ARG;
+    }
+    // (the scaled copy of a product's cotangent is scaled by the very vector the product was formed with)
+    if (c.scaled && c.col_factor != p.scale_src) p.factor_src = c.col_factor, p.factor_slot = p.n_slots++;
+    // (lanes past the last vector read what follows their slot: only results that are masked or dropped see it)
+    p.lds_pitch = static_cast<int>(nv) * V;
+    const size_t lds = (static_cast<size_t>(p.n_slots - 1) * p.lds_pitch + static_cast<size_t>(wr) * 64 * j * V) * sizeof(T);
+    if (lds > kLseRowsMaxLds) {
+        set_error("lse_rows: %d column vectors of %lld elements do not fit the LDS", p.n_slots, (long long)c.cols);
+        return AGMI_ERR_UNSUPPORTED;
+    }
+    const int64_t tiles = ceil_div(c.rows, nw / wr);
+    int blocks = static_cast<int>(std::min<int64_t>(tiles, kLseRowsMaxBlocks));
+    const bool staged = c.col_sums != nullptr && blocks > 1;
+    if (staged) {
+        const int64_t fit = workspace ? static_cast<int64_t>(workspace_bytes / (static_cast<size_t>(c.cols) * sizeof(T))) : 0;
+        blocks = static_cast<int>(std::min<int64_t>(blocks, std::max<int64_t>(fit, 1)));
+    }
+    p.col_out = blocks > 1 ? workspace : c.col_sums;
+    set_kernel_name("lse_cotangent_tile_rows<%s,%d,%d%s%s%s%s>[%lldx%lld]", sizeof(T) == 4 ? "f32" : "f64", wr, j, ans_out ? ",ans" : "",
+                    c.scaled ? ",scaled" : "", c.row_sums ? ",rowsum" : "", c.col_sums ? ",colsum" : "", (long long)c.rows,
+                    (long long)c.cols);
+    const bool cols = c.col_sums != nullptr;
+    probe_begin(s);
+    int rc = AGMI_ERR_UNSUPPORTED;
+    if (wr == 1 && j == 1) rc = launch_lse_rows_kernel<T, 16, 1, 1>(p, cols, blocks, lds, s);
+    else if (wr == 1) rc = launch_lse_rows_kernel<T, 16, 1, 2>(p, cols, blocks, lds, s);
+    else if (wr == 2) rc = launch_lse_rows_kernel<T, 16, 2, 2>(p, cols, blocks, lds, s);
+    else if (wr == 4 && j == 1) rc = launch_lse_rows_kernel<T, 16, 4, 1>(p, cols, blocks, lds, s);
+    else if (wr == 4 && j == 2) rc = launch_lse_rows_kernel<T, 16, 4, 2>(p, cols, blocks, lds, s);
+    else if (wr == 16 && j == 2) rc = launch_lse_rows_kernel<T, 16, 16, 2>(p, cols, blocks, lds, s);
+    else if (wr == 16 && j == 8) rc = launch_lse_rows_kernel<T, 16, 16, 8>(p, cols, blocks, lds, s);
+    else if (wr == 8 && j == 2) rc = launch_lse_rows_kernel<T, 16, 8, 2>(p, cols, blocks, lds, s);
+    else if constexpr (kWide) rc = launch_lse_rows_kernel<T, 8, 8, 8>(p, cols, blocks, lds, s);
+    else rc = launch_lse_rows_kernel<T, 16, 16, 4>(p, cols, blocks, lds, s);
+    probe_end(s);
+    if (rc) return rc;
+    if (cols && blocks > 1) {
+        const int col_blocks = static_cast<int>(ceil_div(c.cols, 64));
+        hipLaunchKernelGGL(lse_cotangent_finish<T>, dim3(static_cast<unsigned>(col_blocks)), dim3(kFinishThreads), 0, s,
+                           static_cast<const T *>(workspace), blocks, c.cols, static_cast<T *>(c.col_sums), col_blocks,
+                           static_cast<const T *>(nullptr), 0, static_cast<int64_t>(0), static_cast<T *>(nullptr));
+        return hip_check(hipGetLastError(), "lse_rows finish launch");
+    }
+    return 0;
+}
+
 }  // namespace agmi
 
 using namespace agmi;
@@ -382,5 +771,30 @@ extern "C" int agmi_lse_cotangent_fused(int dtype, const agmi_lse_cotangent *c, 
     if (dtype == AGMI_F32) return launch_lse_cotangent<float>(*c, workspace, workspace_bytes, s);
     if (dtype == AGMI_F64) return launch_lse_cotangent<double>(*c, workspace, workspace_bytes, s);
     set_error("lse_cotangent: dtype %d is not a floating type", dtype);
+    return AGMI_ERR_ARG;
+}
+
+extern "C" int agmi_lse_rows_fused(int dtype, const agmi_lse_cotangent *c, void *ans, int64_t ans_stride, void *workspace,
+                                   size_t workspace_bytes, void *stream) {
+    if (!c) {
+        set_error("lse_rows: null descriptor");
+        return AGMI_ERR_ARG;
+    }
+    if (c->rows < 0 || c->cols < 0) {
+        set_error("lse_rows: negative extent");
+        return AGMI_ERR_ARG;
+    }
+    if (c->rows == 0 || c->cols == 0) {
+        set_error("lse_rows: no elements");
+        return AGMI_ERR_UNSUPPORTED;
+    }
+    if (!c->x || !c->g) {
+        set_error("lse_rows: null operand");
+        return AGMI_ERR_ARG;
+    }
+    hipStream_t s = as_stream(stream);
+    if (dtype == AGMI_F32) return launch_lse_rows<float>(*c, ans, ans_stride, workspace, workspace_bytes, s);
+    if (dtype == AGMI_F64) return launch_lse_rows<double>(*c, ans, ans_stride, workspace, workspace_bytes, s);
+    set_error("lse_rows: dtype %d is not a floating type", dtype);
     return AGMI_ERR_ARG;
 }

@@ -488,16 +488,18 @@ class LseCotangent(DevArray):
     sums (an offset that was broadcast along the rows), its product with a factor that was broadcast
     down the columns, the column sums of its product with the matrix the factor multiplied.  Each such
     consumer (``row_sums`` / ``scaled_by`` / ``col_sums_with``) gets a :class:`FusedResult`, whose memory
-    exists but whose values do not yet; the first time any of them is read, ONE kernel
-    (``agmi_lse_cotangent_fused``) walks ``x``'s storage once and produces all of them, and this
-    matrix itself never reaches memory.  Anything else reads ``_t`` as on any ``DevArray`` and gets it
-    written out by the elementwise rule kernel.
+    exists but whose values do not yet; the first time any of them is read, ONE kernel walks ``x``'s storage
+    once and produces all of them, and this matrix itself never reaches memory.  Under ``grad`` the logsumexp's
+    own value has usually not run either (``special.logsumexp`` leaves it pending while a trace is open): the same pass
+    forms it (``agmi_lse_rows_fused``; rows too long for that kernel: the reduction, then ``agmi_lse_cotangent_fused``).
+    Anything else reads ``_t`` as on any ``DevArray`` and gets the matrix written out.
     """
 
-    __slots__ = ("_g", "_x", "_ans", "_shape", "_wanted")
+    __slots__ = ("_g", "_x", "_ans", "_ans_kept", "_shape", "_wanted")
 
-    def __init__(self, g_k, x, ans_k, dtype):
-        self._g, self._x, self._ans = g_k, x, ans_k
+    def __init__(self, g_k, x, ans, dtype):
+        self._g, self._x, self._ans = g_k, x, ans
+        self._ans_kept = None  # (rows, 1) form of `ans` once it has a value
         self._shape = x.shape
         self.dtype = dtype
         self._borrowed = False
@@ -506,28 +508,60 @@ class LseCotangent(DevArray):
     def __getattr__(self, name):
         if name != "_t":
             raise AttributeError(name)
-        self.run()
-        self._t = out = map_op(Op.LSE_VJP, self.dtype, self._g, 1.0, self._x, self._ans)._t
+        if self._wanted:
+            self.run()
+        out = _lib.empty(self._shape, self.dtype)
+        if not self._one_pass(scaled=out):
+            out = map_op(Op.LSE_VJP, self.dtype, self._g, 1.0, self._x, DevArray(self._ans_tensor(), self.dtype))._t
+        self._t = out
         return out
 
+    def _ans_tensor(self):
+        kept = self._ans_kept
+        if kept is None:
+            kept = self._ans_kept = self._ans._t.reshape(self._shape[0], 1)
+        return kept
+
+    def _one_pass(self, **wanted):
+        """Everything asked for, and the logsumexp where it has not run, in one pass over ``x``; False: nothing has run."""
+        x, ans = self._x, self._ans
+        pending = type(ans) is PendingReduce and not _has_value(ans)
+        value = _lib.empty((self._shape[0], 1), self.dtype) if pending else None
+        operand = x._affine() if type(x) is LazyDevArray else x._t
+        if not _lib.lse_rows(_lib.DTYPE_CODE[self.dtype], operand, self._g._t, ans=value, **wanted):
+            return False
+        if pending:
+            ans.computed_as(value)
+        return True
+
     @staticmethod
-    def eligible(g_k, x, ans_k, dtype):
-        """The layouts the fused kernel covers: a row-major matrix (its pending map, if any, made of
-        row or column vectors) reduced along its rows; everything in one floating dtype."""
-        if dtype not in _FLOATS or x.dtype != dtype or x.ndim != 2 or type(x) not in (DevArray, LazyDevArray):
+    def takes(x):
+        """Whether the fused kernels cover the operand: a row-major matrix whose pending map, if any, is made of row or
+        column vectors."""
+        dtype = x.dtype
+        if dtype not in _FLOATS or x.ndim != 2 or type(x) not in (DevArray, LazyDevArray):
             return False
         h = x._h()
+        rows, cols = h.shape
+        if rows == 0 or cols == 0 or (h.stride(1) != 1 and cols != 1):
+            return False
         vec = 16 // dtype.itemsize
-        if h.shape[0] == 0 or h.shape[1] == 0 or h.shape[1] % vec or h.stride(1) != 1:
+        if cols % vec and cols > _lib.LSE_ROWS_MAX_VECTORS * vec:
             return False
         if type(x) is LazyDevArray:
             for aux in (x._ascale, x._shift):
                 if isinstance(aux, torch.Tensor) and not (aux.stride(1) == 0 or (aux.stride(1) == 1 and aux.stride(0) == 0)):
                     return False
-        for v in (g_k, ans_k):
-            if type(v) is not DevArray or v.dtype != dtype or v.shape != (h.shape[0], 1):
-                return False
         return True
+
+    @staticmethod
+    def eligible(g_k, x, ans, dtype):
+        """Whether the cotangent of the rows of ``x`` can stay unwritten: everything in one floating dtype, a layout the
+        fused kernels cover, a logsumexp that has run or is pending as a reduction."""
+        if x.dtype != dtype or type(g_k) is not DevArray or g_k.dtype != dtype or not LseCotangent.takes(x):
+            return False
+        rows = x.shape[0]
+        return g_k.shape == (rows, 1) and type(ans) in (DevArray, PendingReduce) and ans.dtype == dtype and ans.shape in ((rows,), (rows, 1))
 
     def computed(self):
         return _has_value(self)
@@ -567,15 +601,16 @@ class LseCotangent(DevArray):
         wanted, self._wanted = self._wanted, {}
         if not wanted:
             return
-        x = self._x
-        operand = x._affine() if type(x) is LazyDevArray else x._t
         rs = wanted.get("row_sums")
         sc = wanted.get("scaled")
         cs = wanted.get("col_sums")
-        ok = _lib.lse_cotangent(_lib.DTYPE_CODE[self.dtype], operand, self._ans._t, self._g._t,
-                                row_sums=rs[1] if rs else None, col_factor=sc[0] if sc else None,
-                                scaled=sc[1] if sc else None, col_sums=cs[1] if cs else None)
-        if ok:
+        outs = dict(row_sums=rs[1] if rs else None, col_factor=sc[0] if sc else None, scaled=sc[1] if sc else None,
+                    col_sums=cs[1] if cs else None)
+        if self._one_pass(**outs):
+            return
+        x = self._x
+        operand = x._affine() if type(x) is LazyDevArray else x._t
+        if _lib.lse_cotangent(_lib.DTYPE_CODE[self.dtype], operand, self._ans_tensor(), self._g._t, **outs):
             return
         # a layout the fused kernel does not take after all: write the matrix out, then the plain kernels
         full = DevArray(self._t, self.dtype)
@@ -1233,6 +1268,11 @@ class PendingReduce(DevArray):
         self._t = out = _map_reduce_now(*self._call)._t
         self._call = None
         return out
+
+    def computed_as(self, value):
+        """Its value has been formed by another kernel, in the tensor ``value`` (any shape of this many elements)."""
+        self._t = value.reshape(self._shape)
+        self._call = None
 
     @property
     def shape(self):

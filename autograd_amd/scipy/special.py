@@ -17,6 +17,7 @@ from ..numpy import devarray as D
 from ..numpy import fusion
 from ..numpy import wrapper as np
 from ..numpy.vjps import _concrete, repeat_to_match_shape
+from ..tracer import trace_stack
 
 
 @primitive
@@ -31,6 +32,11 @@ def logsumexp(x, axis=None, b=1.0, keepdims=False):
             # subtraction and the rule g * exp(x - ans), and a program forms the logsumexp of a short row itself
             # (bit for bit the reduction kernel's value).  So nothing runs here; a reader of the value itself runs it.
             return D.PendingReduce((Op.COPY, Red.LOGSUMEXP, dt, (D._kept(x),), axes, True, None), (x.shape[0], 1), dt)
+        if axes == (1,) and x.dtype == dt and trace_stack.top >= 0 and _rows_in_one_pass(x, keepdims):
+            # Rows of a matrix while a trace is open: the rule's own pass over x forms the value as well (LseCotangent),
+            # so it waits for that pass; anything that reads it first runs the reduction.
+            return D.PendingReduce((Op.COPY, Red.LOGSUMEXP, dt, (D._kept(x),), axes, keepdims, None),
+                                   (x.shape[0], 1) if keepdims else (x.shape[0],), dt)
         return D.map_reduce(Op.COPY, Red.LOGSUMEXP, dt, (x,), axes, keepdims)
     # weighted form, the way scipy evaluates it: m = max(x), log(sum(b * exp(x - m))) + m, with weights of either
     # sign (a negative total gives NaN, as there).  Two passes over x: the maximum, then the weighted sum
@@ -48,6 +54,15 @@ def logsumexp(x, axis=None, b=1.0, keepdims=False):
     if keepdims:
         return out
     return np.reshape.fun(out, tuple(n for d, n in enumerate(x.shape) if d not in axes))
+
+
+def _rows_in_one_pass(x, keepdims):
+    """Whether the rows of ``x`` go to the kernels that form their logsumexp and its cotangent together.  Short rows with
+    the axis kept (a log-softmax) belong to the chains around them instead, which form the value themselves.  Below 8192
+    elements (launches, not bytes, are the cost there: 20 us against 25 replayed even at 300 x 250) the separate kernels
+    stay, so that small programs keep the bits of their rule-by-rule evaluation; the pass rescales each exponential
+    where the rule subtracts the logsumexp first."""
+    return x.size >= 8192 and D.LseCotangent.takes(x) and not (keepdims and fusion.rows_fit_a_wave(x.shape, x.dtype))
 
 
 def _keep(a, shape, axis, keepdims):
@@ -71,13 +86,13 @@ def _make_grad_logsumexp(ans, x, axis=None, b=1.0, keepdims=False):
             return g_repeated * b * np.exp(x - ans_kept)
         if _concrete(g, ans, x, b):
             g_k = _keep(D.asarray(g), shape, axis, keepdims)
-            ans_k = _keep(ans, shape, axis, keepdims)
-            dt = D._float_dtype(D.result_dtype(g_k, x, ans_k))
+            dt = D._float_dtype(D.result_dtype(g_k, x, ans))
             if (type(b) is float and b == 1.0 and len(shape) == 2 and D.normalize_axes(axis, 2) == (1,)
-                    and D.LseCotangent.eligible(g_k, x, ans_k, dt)):
+                    and _rows_in_one_pass(x, keepdims) and D.LseCotangent.eligible(g_k, x, ans, dt)):
                 # rows of a matrix: the cotangent stays unwritten until its consumers are known; the usual
                 # ones (row sums, a rescaled copy, column sums of a product) then come out of one pass
-                return D.LseCotangent(g_k, x, ans_k, dt)
+                return D.LseCotangent(g_k, x, ans, dt)
+            ans_k = _keep(ans, shape, axis, keepdims)
             return D.map_op(Op.LSE_VJP, dt, g_k, b, x, ans_k)
         g_repeated, _ = repeat_to_match_shape(g, shape, dtype, axis, keepdims)
         ans_repeated, _ = repeat_to_match_shape(ans, shape, dtype, axis, keepdims)

@@ -353,6 +353,14 @@ typedef struct agmi_lse_cotangent {
 int agmi_lse_cotangent_fused(int dtype, const agmi_lse_cotangent *c, void *workspace, size_t workspace_bytes,
                              void *stream);
 
+/* The same results (and the logsumexp itself) in one pass over the operand, for a logsumexp that has not run: ans[r *
+ * ans_stride] (may be NULL) is written, c->ans is not read.  Any number of columns up to 4096 vectors of 16 bytes (16384 float32,
+ * 8192 float64) at any element alignment, and up to twice that where it is no whole number of vectors; col_factor NULL means a factor of one (`scaled` is then S itself).  Column sums
+ * are staged per block (at most 256 rows of `cols` elements) in `workspace`; a smaller workspace means fewer blocks.
+ * AGMI_ERR_UNSUPPORTED outside this. */
+int agmi_lse_rows_fused(int dtype, const agmi_lse_cotangent *c, void *ans, int64_t ans_stride, void *workspace,
+                        size_t workspace_bytes, void *stream);
+
 /* C[m,n] = alpha * sum_k A[m,k] B[k,n] + beta * C[m,n] on the matrix cores (MFMA), dtype
  * AGMI_F32 or AGMI_F64.  A and B are addressed as A[m*a_rs + k*a_cs], B[k*b_rs + n*b_cs], so
  * the transposed operands of the adjoints need no copy; C is row-major with leading

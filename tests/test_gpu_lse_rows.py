@@ -1,0 +1,132 @@
+"""``agmi_lse_rows_fused``: a row-wise logsumexp, its cotangent and what consumes it in one pass over the operand.
+
+Sizes sit at the edges of the kernel's variants (64 ... 8192 vectors of 16 bytes to a row, one more and one less) and at numbers
+of rows that leave blocks and row groups part empty; the oracle is NumPy in float64.
+"""
+
+import numpy as onp
+import pytest
+import scipy.special
+
+pytestmark = pytest.mark.gpu
+
+F32, F64 = onp.float32, onp.float64
+# (vectors to a row, what is added to the elements they hold, rows)
+EDGES = [(1, -1, 3), (1, 0, 33), (64, -1, 5), (64, 1, 700), (128, 0, 2500), (128, 1, 2049), (256, -1, 2100), (256, -3, 70), (256, 1, 9),
+         (512, 1, 1100), (1024, 0, 1030), (1024, -1, 300), (1024, 1, 37), (2048, 1, 261), (4096, 0, 5), (4096, 1, 300), (8192, -1, 3)]
+
+
+def _tolerance(dtype, cols):
+    # x - ans is rounded before the exponential (|x - ans| < 32 here: 32 half-ulps of relative error at most), sums add
+    # a handful of roundings on top
+    return 64 * onp.finfo(dtype).eps
+
+
+@pytest.mark.parametrize("dtype", [F32, F64])
+@pytest.mark.parametrize("vectors,extra,rows", EDGES)
+def test_every_result_at_the_edges_of_the_variants(dtype, vectors, extra, rows):
+    import torch
+
+    from autograd_amd import _lib
+
+    cols = vectors * (16 // onp.dtype(dtype).itemsize) + extra
+    rs = onp.random.RandomState(cols + rows)
+    dev, code = _lib.device(), _lib.DTYPE_CODE[onp.dtype(dtype)]
+    pitch = cols + 3  # rows of the operand and of the copy lie apart: what is between them is not touched
+    mem = rs.randn(rows, pitch).astype(dtype)
+    by_col, by_row, g = rs.uniform(0.5, 1.5, cols).astype(dtype), rs.randn(rows, 1).astype(dtype), rs.uniform(0.5, 2.0, (rows, 1)).astype(dtype)
+    put = lambda a: torch.from_numpy(onp.ascontiguousarray(a)).to(dev)
+    t_mem = put(mem)[:, :cols]
+    t_col, t_row, t_g = put(by_col), put(by_row), put(g)
+    wide = lambda t: t.expand(rows, cols)
+    forms = {
+        "A*b + c": (_lib.Affine(t_mem, 1.0, wide(t_row), wide(t_col)), mem[:, :cols].astype(F64) * by_col + by_row),
+        "-A + b": (_lib.Affine(t_mem, -1.0, wide(t_col)), -mem[:, :cols].astype(F64) + by_col),
+        "A": (t_mem, mem[:, :cols].astype(F64)),
+    }
+    tol = _tolerance(dtype, cols)
+    for name, (operand, x) in forms.items():
+        ans = scipy.special.logsumexp(x, axis=1, keepdims=True)
+        S = g.astype(F64) * onp.exp(x - ans)
+        for factor in (t_col, None):
+            kind = dict(dtype=t_mem.dtype, device=dev)
+            out = torch.full((rows, pitch), 7.0, **kind)
+            t_ans, row_sums, col_sums = torch.empty((rows, 1), **kind), torch.empty((rows, 1), **kind), torch.empty((1, cols), **kind)
+            if not _lib.lse_rows(code, operand, t_g, ans=t_ans, row_sums=row_sums, col_factor=factor, scaled=out[:, :cols], col_sums=col_sums):
+                assert vectors > 3000, name  # (two or three vectors along the longest rows do not fit the LDS)
+                continue
+            want = S * by_col if factor is not None else S
+            got = out.cpu().numpy()
+            assert onp.all(got[:, cols:] == 7.0), name
+            for what, have, ref in (("copy", got[:, :cols], want), ("ans", t_ans.cpu().numpy(), ans),
+                                    ("row sums", row_sums.cpu().numpy(), S.sum(1, keepdims=True)),
+                                    ("column sums", col_sums.cpu().numpy(), (mem[:, :cols] * S).sum(0, keepdims=True))):
+                scale = onp.abs(mem[:, :cols] * S).sum(0, keepdims=True) if what == "column sums" else onp.maximum(onp.abs(ref), tol)
+                assert onp.all(onp.abs(have - ref) <= tol * scale), (name, what, factor is None)
+            # each result on its own, too (other instantiations)
+            alone = torch.empty((rows, cols), **kind)
+            assert _lib.lse_rows(code, operand, t_g, col_factor=factor, scaled=alone)
+            assert onp.array_equal(alone.cpu().numpy(), got[:, :cols]), name
+            if not _lib.lse_rows(code, operand, t_g, col_sums=(again := torch.empty_like(col_sums))):
+                assert vectors > 3000, name
+                continue
+            assert torch.equal(again, col_sums), name
+
+
+@pytest.mark.parametrize("dtype", [F32, F64])
+@pytest.mark.parametrize("cols", [7, 600, 5000, 16001])
+def test_rows_with_infinities_and_nans(dtype, cols):
+    """Special values travel as through the two separate kernels (scipy's logsumexp, then g * exp(x - ans))."""
+    import torch
+
+    from autograd_amd import _lib
+
+    rs = onp.random.RandomState(cols)
+    dev, code = _lib.device(), _lib.DTYPE_CODE[onp.dtype(dtype)]
+    x = rs.randn(12, cols).astype(dtype)
+    x[1], x[2, 3], x[3, 0], x[4, cols - 1], x[5] = -onp.inf, onp.inf, onp.nan, -onp.inf, onp.nan
+    x[6, 1], x[6, 2] = onp.inf, onp.nan
+    x[7] = -onp.inf
+    x[7, cols // 2] = -1000.0
+    x[8, :] = 80.0
+    x[9, : cols // 2] = -onp.inf
+    t_x, t_g = torch.from_numpy(x).to(dev), torch.full((12, 1), 2.0, dtype=torch.float32 if dtype is F32 else torch.float64, device=dev)
+    t_ans, row_sums, out = torch.empty_like(t_g), torch.empty_like(t_g), torch.empty_like(t_x)
+    assert _lib.lse_rows(code, t_x, t_g, ans=t_ans, row_sums=row_sums, scaled=out)
+    with onp.errstate(all="ignore"):
+        m = onp.max(x.astype(F64), axis=1, keepdims=True)
+        safe = onp.where(onp.isfinite(m), m, 0.0)
+        ans = onp.log(onp.sum(onp.exp(x.astype(F64) - safe), axis=1, keepdims=True)) + safe
+        S = 2.0 * onp.exp(x.astype(F64) - ans)
+    for have, ref in ((t_ans, ans), (out, S), (row_sums, S.sum(1, keepdims=True))):
+        have = have.cpu().numpy().astype(F64)
+        assert onp.array_equal(onp.isnan(have), onp.isnan(ref)) and onp.array_equal(onp.isinf(have), onp.isinf(ref))
+        fine = onp.isfinite(ref)
+        # (80 and -1000 bring the error of |ans| ulps that rounding ans leaves in exp(x - ans))
+        assert onp.all(onp.abs(have[fine] - ref[fine]) <= 2048 * onp.finfo(dtype).eps * onp.maximum(onp.abs(ref[fine]), 1e-30))
+
+
+def test_a_pending_logsumexp_is_formed_by_the_pass_that_differentiates_it():
+    import autograd_amd as ag
+    import autograd_amd.numpy as dnp
+    from autograd_amd import _lib
+    from autograd_amd.scipy.special import logsumexp
+
+    rs = onp.random.RandomState(3)
+    a, b, c = rs.randn(301, 1003), rs.uniform(0.5, 1.5, 1003), rs.randn(301)
+    A, B, C = (dnp.asarray(v) for v in (a, b, c))
+    f = lambda A, B, C: dnp.sum(logsumexp(A * B[None, :] + C[:, None], axis=1) ** 2)
+    g = lambda A, B, C: dnp.sum(logsumexp(A * B[None, :] + C[:, None], axis=1))
+    x = a * b + c[:, None]
+    lse = scipy.special.logsumexp(x, axis=1, keepdims=True)
+    S = onp.exp(x - lse)
+    with _lib.KernelTimer() as kt:
+        dA, dB, dC = ag.grad(g, (0, 1, 2))(A, B, C)
+    assert sum(row["launches"] for row in kt.summary().values()) == 1
+    for have, ref in ((dA, S * b), (dB, (a * S).sum(0)), (dC, S.sum(1))):
+        assert onp.allclose(have.numpy(), ref, rtol=1e-12, atol=1e-12)
+    value, dA = ag.value_and_grad(f)(A, B, C)  # a reader of the value first: the reduction runs, the rule finds it
+    assert onp.allclose(float(value), (lse**2).sum(), rtol=1e-13)
+    assert onp.allclose(dA.numpy(), 2 * lse * S * b, rtol=1e-12, atol=1e-12)
+    untraced = logsumexp(A, axis=1)
+    assert type(untraced).__name__ == "DevArray"
