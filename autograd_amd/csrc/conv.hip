@@ -15,10 +15,9 @@
 // multiply-adds whose filter operands are wave-uniform.
 //
 // correlate_reduce: the filter's cotangent has few outputs (channels x channels x window) and a
-// reduction over batch x image.  A block owns one output; its 256 lanes split the contracted
-// axis and the innermost window axis between them (so neighbouring lanes read neighbouring
-// elements of both operands), walk the other window axes in nested loops, and combine in LDS in
-// a fixed tree order.
+// reduction over batch x image.  A block owns a small tile of outputs; its lanes split the contracted
+// axis and the window between them (neighbouring lanes along the innermost window axis, so that they read
+// neighbouring elements of both operands), and combine in a fixed tree order.
 #include "common.h"
 
 namespace agmi {
@@ -31,7 +30,9 @@ struct CorrParams {
     int64_t o_fs, o_ss, o_s[3];
     uint32_t p_total;    // P[0] * P[1] * P[2]
     uint32_t tiles;      // correlate_positions: blocks per filter-batch tile
-    uint32_t lane_bits;  // correlate_reduce: log2 of the lanes that share the innermost window axis
+    // correlate_reduce: log2 of the lanes that share the innermost window axis and the contracted axis (the rest of the
+    // block shares the window's rows), threads in a block
+    int lane_bits, d_bits, threads;
     // correlate_tiled: a block covers 2^jt_bits images x 2^p1_bits rows x 2^p2_bits columns of output
     // (256 positions) and stages the H x W window of signal they read, per image, in LDS
     int jt_bits, p1_bits, p2_bits, H, W;
@@ -41,6 +42,7 @@ struct CorrParams {
 };
 
 constexpr int kTileLoads = 8;    // signal elements a thread stages per step: tiles of up to 2048 elements
+constexpr int kReduceBlock = 1024;  // most threads a block of correlate_reduce has
 constexpr int kFilterLoads = 4;  // filter elements a thread stages per step: DT * K1 * K2 * TI up to 1024
 
 template <typename T>
@@ -260,64 +262,117 @@ __global__ __launch_bounds__(kBlock) void correlate_tiled(const T *__restrict__ 
         if (i0 + t < c.I) o[(i0 + t) * c.o_fs] = acc[t];
 }
 
-template <typename T>
-__global__ __launch_bounds__(kBlock) void correlate_reduce(const T *__restrict__ filter, const T *__restrict__ signal,
-                                                           T *__restrict__ out, const CorrParams c) {
+// The filter's cotangent.  A block owns TI filter-batch entries x PT neighbouring positions along the innermost axis; its
+// threads split the window's columns, the contracted axis and (where that is short) the window's rows, and every TI + PT
+// loads feed TI * PT multiply-adds: at one output per block the cache's bandwidth bounds a problem of many outputs, and the
+// latency of a thread's own serial chain one of few, hence blocks of up to 1024 threads.  PT > 1 only where every tap of
+// the innermost axis meets the signal; entries and positions past the last repeat it (computed, never stored).
+// Measured (float64, batch 256, 5 x 5 windows, against one output per block of 256): 6 -> 16 channels of 12 x 12 images
+// (2400 outputs) 43 -> 21 us, 1 -> 6 channels of 28 x 28 (150 outputs, too few for tiles: the chain's loads still bound it)
+// 77 -> 50 us.
+template <typename T, int TI, int PT>
+__global__ __launch_bounds__(kReduceBlock) void correlate_reduce(const T *__restrict__ filter, const T *__restrict__ signal,
+                                                                 T *__restrict__ out, const CorrParams c) {
+    const uint32_t n_p2 = (static_cast<uint32_t>(c.P[2]) + PT - 1) / PT, n_i = (static_cast<uint32_t>(c.I) + TI - 1) / TI;
     uint32_t q = blockIdx.x;
-    const int64_t p2 = q % static_cast<uint32_t>(c.P[2]);
-    q /= static_cast<uint32_t>(c.P[2]);
+    const int64_t p2 = static_cast<int64_t>(q % n_p2) * PT;
+    q /= n_p2;
     const int64_t p1 = q % static_cast<uint32_t>(c.P[1]);
     q /= static_cast<uint32_t>(c.P[1]);
     const int64_t p0 = q % static_cast<uint32_t>(c.P[0]);
     q /= static_cast<uint32_t>(c.P[0]);
-    const int64_t i = q % static_cast<uint32_t>(c.I), j = q / static_cast<uint32_t>(c.I);
-    const int64_t lanes_k = int64_t(1) << c.lane_bits, lanes_d = kBlock >> c.lane_bits;
-    const int64_t lk = threadIdx.x & (lanes_k - 1), ld = threadIdx.x >> c.lane_bits;
-    const T *f = filter + i * c.f_bs;
-    const T *s = signal + j * c.s_bs;
+    const int64_t i0 = static_cast<int64_t>(q % n_i) * TI, j = q / n_i;
+    const int tid = threadIdx.x;
+    const int lanes_k = 1 << c.lane_bits, lanes_d = 1 << c.d_bits, lanes_1 = blockDim.x >> (c.lane_bits + c.d_bits);
+    const int lk = tid & (lanes_k - 1), ld = tid >> c.lane_bits & (lanes_d - 1), l1 = tid >> (c.lane_bits + c.d_bits);
     const int64_t b0 = p0 - c.pad[0], b1 = p1 - c.pad[1], b2 = p2 - c.pad[2];
+    int64_t f_off[TI], s_off[PT];
+#pragma unroll
+    for (int t = 0; t < TI; ++t) f_off[t] = (i0 + t < c.I ? i0 + t : c.I - 1) * c.f_bs;
+#pragma unroll
+    for (int u = 0; u < PT; ++u) s_off[u] = (p2 + u < c.P[2] ? u : c.P[2] - 1 - p2) * c.s_s[2];
     // The window rows that meet the signal are found up front (the position is the same for the whole block),
-    // so the inner loop is free of bounds tests and the loads of four rows are issued together.
-    T acc0 = T(0), acc1 = T(0);
+    // so the inner loop is free of bounds tests and the loads of several rows are issued together.
+    T acc[TI][PT];
+#pragma unroll
+    for (int t = 0; t < TI; ++t)
+#pragma unroll
+        for (int u = 0; u < PT; ++u) acc[t][u] = T(0);
     const int64_t lo = b1 < 0 ? -b1 : 0;                                     // k1 in [lo, hi)
     const int64_t hi = c.N[1] - b1 < c.K[1] ? c.N[1] - b1 : c.K[1];
+    const int64_t f_row = lanes_1 * c.f_s[1], s_row = lanes_1 * c.s_s[1];
+#pragma unroll 1
     for (int64_t k2 = lk; k2 < c.K[2]; k2 += lanes_k) {
         const int64_t s2 = b2 + k2;
         if (static_cast<uint64_t>(s2) >= static_cast<uint64_t>(c.N[2])) continue;
-        const T *f2 = f + k2 * c.f_s[2];
-        const T *sg2 = s + s2 * c.s_s[2] + b1 * c.s_s[1];
+        const T *f2 = filter + k2 * c.f_s[2] + (lo + l1) * c.f_s[1];
+        const T *sg2 = signal + j * c.s_bs + s2 * c.s_s[2] + (b1 + lo + l1) * c.s_s[1];
+#pragma unroll 1
         for (int64_t d = ld; d < c.D; d += lanes_d) {
+#pragma unroll 1
             for (int64_t k0 = 0; k0 < c.K[0]; ++k0) {
                 const int64_t s0 = b0 + k0;
                 if (static_cast<uint64_t>(s0) >= static_cast<uint64_t>(c.N[0])) continue;
                 const T *fr = f2 + d * c.f_ds + k0 * c.f_s[0];
                 const T *sr = sg2 + d * c.s_ds + s0 * c.s_s[0];
-                int64_t k1 = lo;
-                for (; k1 + 4 <= hi; k1 += 4) {
-                    const T fa = fr[k1 * c.f_s[1]], fb = fr[(k1 + 1) * c.f_s[1]];
-                    const T fc = fr[(k1 + 2) * c.f_s[1]], fe = fr[(k1 + 3) * c.f_s[1]];
-                    const T sa = sr[k1 * c.s_s[1]], sb = sr[(k1 + 1) * c.s_s[1]];
-                    const T sc = sr[(k1 + 2) * c.s_s[1]], se = sr[(k1 + 3) * c.s_s[1]];
-                    acc0 = fused_mul_add(fa, sa, acc0);
-                    acc1 = fused_mul_add(fb, sb, acc1);
-                    acc0 = fused_mul_add(fc, sc, acc0);
-                    acc1 = fused_mul_add(fe, se, acc1);
+                constexpr int U = TI * PT == 1 ? 4 : 1;  // rows in flight (more of them spill the 128 registers)
+                int64_t k1 = lo + l1;
+#pragma unroll 1
+                for (; k1 + (U - 1) * lanes_1 < hi; k1 += U * lanes_1) {
+                    T fv[U][TI], sv[U][PT];
+#pragma unroll
+                    for (int m = 0; m < U; ++m) {
+#pragma unroll
+                        for (int t = 0; t < TI; ++t) fv[m][t] = fr[f_off[t] + m * f_row];
+#pragma unroll
+                        for (int u = 0; u < PT; ++u) sv[m][u] = sr[s_off[u] + m * s_row];
+                    }
+#pragma unroll
+                    for (int m = 0; m < U; ++m)
+#pragma unroll
+                        for (int t = 0; t < TI; ++t)
+#pragma unroll
+                            for (int u = 0; u < PT; ++u) acc[t][u] = fused_mul_add(fv[m][t], sv[m][u], acc[t][u]);
+                    fr += U * f_row;
+                    sr += U * s_row;
                 }
-                for (; k1 < hi; ++k1) acc0 = fused_mul_add(fr[k1 * c.f_s[1]], sr[k1 * c.s_s[1]], acc0);
+                if constexpr (U == 1) continue;
+#pragma unroll 1
+                for (; k1 < hi; k1 += lanes_1) {
+                    T fv[TI], sv[PT];
+#pragma unroll
+                    for (int t = 0; t < TI; ++t) fv[t] = fr[f_off[t]];
+#pragma unroll
+                    for (int u = 0; u < PT; ++u) sv[u] = sr[s_off[u]];
+#pragma unroll
+                    for (int t = 0; t < TI; ++t)
+#pragma unroll
+                        for (int u = 0; u < PT; ++u) acc[t][u] = fused_mul_add(fv[t], sv[u], acc[t][u]);
+                    fr += f_row;
+                    sr += s_row;
+                }
             }
         }
     }
-    const T acc = acc0 + acc1;
-    __shared__ T partial[kBlock];
-    partial[threadIdx.x] = acc;
+    // combined in a fixed tree order: the lanes of a wave, then the waves of the block
+    __shared__ T partial[kReduceBlock / 64][TI * PT];
+    const int wave = tid >> 6, lane = tid & 63;
+#pragma unroll
+    for (int t = 0; t < TI; ++t)
+#pragma unroll
+        for (int u = 0; u < PT; ++u) {
+            T v = acc[t][u];
+#pragma unroll
+            for (int half = 32; half > 0; half >>= 1) v = v + __shfl_down(v, half, 64);
+            if (lane == 0) partial[wave][t * PT + u] = v;
+        }
     __syncthreads();
-    for (int half = kBlock / 2; half > 0; half >>= 1) {
-        if (static_cast<int>(threadIdx.x) < half)
-            partial[threadIdx.x] = partial[threadIdx.x] + partial[threadIdx.x + half];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
-        out[i * c.o_fs + j * c.o_ss + p0 * c.o_s[0] + p1 * c.o_s[1] + p2 * c.o_s[2]] = partial[0];
+    if (tid >= TI * PT) return;
+    const int t = tid / PT, u = tid - t * PT;
+    if (i0 + t >= c.I || p2 + u >= c.P[2]) return;
+    T v = partial[0][tid];
+    for (int w = 1; w < static_cast<int>(blockDim.x >> 6); ++w) v = v + partial[w][tid];
+    out[(i0 + t) * c.o_fs + j * c.o_ss + p0 * c.o_s[0] + p1 * c.o_s[1] + (p2 + u) * c.o_s[2]] = v;
 }
 
 template <typename T, int TI>
@@ -350,6 +405,40 @@ void launch_tiled(const agmi_correlation *a, CorrParams &c, hipStream_t s) {
     }
 }
 
+template <typename T, int TI, int PT>
+void launch_reduce_tile(const agmi_correlation *a, const CorrParams &c, int64_t blocks, hipStream_t s) {
+    hipLaunchKernelGGL((correlate_reduce<T, TI, PT>), dim3(static_cast<unsigned>(blocks)), dim3(c.threads), 0, s,
+                       static_cast<const T *>(a->filter.data), static_cast<const T *>(a->signal.data),
+                       static_cast<T *>(a->out), c);
+}
+
+// The tile of outputs per block: of the tiles that still give about one block per CU (192 of 256), the one with the fewest
+// loads in all.  Tiles along the innermost axis need every tap of it inside the signal.
+template <typename T>
+void launch_reduce(const agmi_correlation *a, const CorrParams &c, hipStream_t s) {
+    const bool inside = c.pad[2] == 0 && c.P[2] + c.K[2] - 1 <= c.N[2];
+    static const int tiles[][2] = {{1, 1}, {2, 1}, {4, 1}, {1, 3}, {2, 3}, {1, 5}, {2, 5}};
+    int best = 0;
+    int64_t best_loads = 0, best_blocks = 0;
+    for (int k = 0; k < static_cast<int>(sizeof(tiles) / sizeof(tiles[0])); ++k) {
+        const int ti = tiles[k][0], pt = tiles[k][1];
+        const int64_t blocks = ceil_div(c.I, ti) * ceil_div(c.P[2], pt) * c.P[0] * c.P[1] * c.J;
+        if (k > 0 && ((pt > 1 && !inside) || blocks < 192 || blocks * (ti + pt) >= best_loads)) continue;
+        best = k;
+        best_blocks = blocks;
+        best_loads = blocks * (ti + pt);
+    }
+    switch (best) {
+        case 0: launch_reduce_tile<T, 1, 1>(a, c, best_blocks, s); break;
+        case 1: launch_reduce_tile<T, 2, 1>(a, c, best_blocks, s); break;
+        case 2: launch_reduce_tile<T, 4, 1>(a, c, best_blocks, s); break;
+        case 3: launch_reduce_tile<T, 1, 3>(a, c, best_blocks, s); break;
+        case 4: launch_reduce_tile<T, 2, 3>(a, c, best_blocks, s); break;
+        case 5: launch_reduce_tile<T, 1, 5>(a, c, best_blocks, s); break;
+        default: launch_reduce_tile<T, 2, 5>(a, c, best_blocks, s); break;
+    }
+}
+
 template <typename T>
 void launch(const agmi_correlation *a, CorrParams &c, int tile, bool tiled, hipStream_t s) {
     if (tiled) {
@@ -363,9 +452,7 @@ void launch(const agmi_correlation *a, CorrParams &c, int tile, bool tiled, hipS
     }
     switch (tile) {
         case 0:
-            hipLaunchKernelGGL((correlate_reduce<T>), dim3(static_cast<unsigned>(c.I * c.J * c.p_total)), dim3(kBlock),
-                               0, s, static_cast<const T *>(a->filter.data), static_cast<const T *>(a->signal.data),
-                               static_cast<T *>(a->out), c);
+            launch_reduce<T>(a, c, s);
             break;
         case 1: launch_positions<T, 1>(a, c, s); break;
         case 2: launch_positions<T, 2>(a, c, s); break;
@@ -458,9 +545,13 @@ extern "C" int agmi_correlate(int dtype, const agmi_correlation *a, void *stream
         if (c.I > cand / 2 && ceil_div(c.I, cand) * pairs >= 65536) tile = cand;
     if (tile == 1 && c.I * pairs < 16384 && r_total >= 64) tile = 0;
     if (tile == 0) {
-        // lanes along the innermost window axis: the power of two that covers it, at most the block
-        c.lane_bits = 0;
+        // blocks of 1024 once a thread of such a block still has four terms; lanes along the innermost window axis: the
+        // power of two that covers it, at most 256; along the contracted axis likewise, at most what is left
+        c.threads = r_total >= 4 * kReduceBlock ? kReduceBlock : kBlock;
+        const int bits = c.threads == kReduceBlock ? 10 : 8;
+        c.lane_bits = c.d_bits = 0;
         while (c.lane_bits < 8 && (int64_t(1) << c.lane_bits) < c.K[2]) ++c.lane_bits;
+        while (c.lane_bits + c.d_bits < bits && (int64_t(1) << c.d_bits) < c.D) ++c.d_bits;
     }
     // The LDS-staged kernel when its tiles fit: 256 positions per block shaped to the output (columns
     // first), the window of signal they read within kTileLoads x 256 elements, the taps within

@@ -161,3 +161,37 @@ def test_pad_and_its_rules_are_exact(dtype):
     assert onp.array_equal(tangent.numpy(), onp.pad(x, 2, mode="constant"))
     with pytest.raises(NotImplementedError):
         dnp.pad(dnp.asarray(x), 1, mode="reflect")
+
+
+# (batch, channels in, channels out, image, window): one block per output with blocks of 256 and of 1024 threads, tiles of
+# outputs with remainders along the channels and the window (widths 1 ... 7), short and long contracted axes
+REDUCTIONS = [(3, 1, 1, (9, 9), (2, 2)), (40, 1, 6, (12, 12), (5, 5)), (33, 6, 16, (9, 10), (5, 5)), (64, 5, 13, (7, 9), (3, 3)),
+              (300, 2, 3, (5, 40), (1, 7)), (17, 8, 24, (6, 6), (4, 4)), (2, 7, 9, (40, 6), (5, 6)), (5, 3, 31, (11, 3), (3, 1))]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize("mode", ["valid", "full"])
+@pytest.mark.parametrize("batch,cin,cout,image,window", REDUCTIONS)
+def test_filter_cotangent_at_the_edges_of_its_tiles(dtype, mode, batch, cin, cout, image, window):
+    """The filter's cotangent is itself a contraction over batch and image: the oracle is that sum in float64."""
+    import autograd_amd as ag
+    import autograd_amd.numpy as dnp
+    from autograd_amd.scipy.signal import convolve as dconv
+
+    rs = onp.random.RandomState(batch + cin + cout)
+    x, w = rs.randn(batch, cin, *image).astype(dtype), rs.randn(cin, cout, *window).astype(dtype)
+    out_shape = [n - k + 1 if mode == "valid" else n + k - 1 for n, k in zip(image, window)]
+    g = rs.randn(batch, cout, *out_shape).astype(dtype)
+    X, G = dnp.array(x), dnp.array(g)
+    dw = ag.grad(lambda W: dnp.sum(dconv(X, W, axes=([2, 3], [2, 3]), dot_axes=([1], [0]), mode=mode) * G))(dnp.array(w)).numpy()
+    pad = [0, 0] if mode == "valid" else [k - 1 for k in window]
+    xp = onp.pad(x.astype("float64"), [(0, 0), (0, 0)] + [(p, p) for p in pad])
+    want, scale = onp.zeros(w.shape), onp.zeros(w.shape)
+    for a in range(window[0]):
+        for b in range(window[1]):
+            part = xp[:, :, window[0] - 1 - a:, window[1] - 1 - b:][:, :, :out_shape[0], :out_shape[1]]
+            want[:, :, a, b] = onp.einsum("bcij,boij->co", part, g.astype("float64"))
+            scale[:, :, a, b] = onp.einsum("bcij,boij->co", abs(part), abs(g.astype("float64")))
+    # a thread's serial chain and the tree above it: at most terms / 256 + 14 roundings of partial sums of |terms|
+    terms = batch * out_shape[0] * out_shape[1]
+    assert (abs(dw - want) <= (terms / 256 + 14 + 2) * onp.finfo(dtype).eps * scale).all()
