@@ -1051,6 +1051,24 @@ static void launch_mode_b(int mode_b, const GemmParams &p, dim3 grid, hipStream_
 
 static const char *mode_name(int m) { return m == kXC ? "x" : (m == kKC ? "k" : "g"); }
 
+// Into how many slices of K a product of few tiles and a long K is cut (2 ... `most`, or 1 if no two fit).  A round of up to
+// 256 blocks, one per CU, takes as long as one slice however full it is, so the time is rounds x slabs per slice: filling
+// the machine once and a little more (88 tiles x 3 = 264 blocks) costs two rounds for the work of one.  The partial tiles
+// are written and read once each; a slab takes about 0.5 us, in which 2 MB of them move.  Measured, float32:
+// 641 x 512 x 16384 in 3 slices 173 us, 513 x 128 x 16384 in 15 slices (18 tiles, 270 blocks) 35 us before this rule.
+static int64_t k_slices(int64_t tiles, int64_t K, int64_t BK, int64_t most, double tile_bytes) {
+    int64_t best = 1;
+    double best_cost = 0.0;
+    for (int64_t s = 2; s <= most && (s == 2 || tiles * s <= 1024); ++s) {
+        const double cost = static_cast<double>(ceil_div(tiles * s, 256) * ceil_div(K, s * BK)) + static_cast<double>(s) * tile_bytes / 1e6;
+        if (best == 1 || cost < best_cost) {
+            best = s;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
 template <class MF, int BM, int BN, int BK, int DEPTH, int KS = 1>
 static int launch_gemm(GemmParams p, int64_t batch, hipStream_t s, void *ws = nullptr, size_t ws_bytes = 0) {
     using T = typename MF::elem_t;
@@ -1072,9 +1090,9 @@ static int launch_gemm(GemmParams p, int64_t batch, hipStream_t s, void *ws = nu
     p.k_per_split = ceil_div(p.K, BK) * BK;
     const int64_t tiles = tm * tn * batch;
     if (ws != nullptr && tiles < 128 && p.K >= 8 * BK) {
-        int64_t splits = std::min<int64_t>(ceil_div(256, tiles), p.K / (4 * BK));
-        splits = std::min<int64_t>(splits, static_cast<int64_t>(ws_bytes / (sizeof(T) * (size_t)(batch * p.M * p.N))));
-        splits = std::min<int64_t>(splits, 64);
+        const size_t result_bytes = sizeof(T) * (size_t)(batch * p.M * p.N);
+        const int64_t most = std::min<int64_t>(std::min<int64_t>(64, p.K / (4 * BK)), static_cast<int64_t>(ws_bytes / result_bytes));
+        const int64_t splits = k_slices(tiles, p.K, BK, most, static_cast<double>(result_bytes));
         if (splits > 1) {
             p.k_per_split = ceil_div(ceil_div(p.K, splits), BK) * BK;
             p.splits = static_cast<int>(ceil_div(p.K, p.k_per_split));
@@ -1133,9 +1151,9 @@ static int launch_direct(GemmParams p, int64_t batch, hipStream_t s, void *ws, s
     p.k_per_split = ceil_div(p.K, BK) * BK;
     const int64_t tiles = tm * tn * batch;
     if (ws != nullptr && tiles < 128 && p.K >= 8 * BK) {  // few tiles, long K: cut K across blocks
-        int64_t splits = std::min<int64_t>(ceil_div(256, tiles), p.K / (4 * BK));
-        splits = std::min<int64_t>(splits, static_cast<int64_t>(ws_bytes / (sizeof(float) * (size_t)(batch * p.M * p.N))));
-        splits = std::min<int64_t>(splits, 64);
+        const size_t result_bytes = sizeof(float) * (size_t)(batch * p.M * p.N);
+        const int64_t most = std::min<int64_t>(std::min<int64_t>(64, p.K / (4 * BK)), static_cast<int64_t>(ws_bytes / result_bytes));
+        const int64_t splits = k_slices(tiles, p.K, BK, most, static_cast<double>(result_bytes));
         if (splits > 1) {
             p.k_per_split = ceil_div(ceil_div(p.K, splits), BK) * BK;
             p.splits = static_cast<int>(ceil_div(p.K, p.k_per_split));
