@@ -534,7 +534,7 @@ extern "C" int agmi_correlate(int dtype, const agmi_correlation *a, void *stream
     c.p_total = static_cast<uint32_t>(p_total);
 
     // Widest filter-batch tile that still leaves four waves per SIMD of position threads; when even
-    // single entries do not give 64 blocks and the reduction is long enough to share, one block per output.
+    // single entries do not give 64 blocks and the reduction is long enough to share, a block per few outputs.
     const int64_t pairs = c.J * p_total;
     if (pairs > 0x7fffffffLL) {
         set_error("correlate: too many output positions for one launch");
