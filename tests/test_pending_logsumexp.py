@@ -1,0 +1,115 @@
+"""A row-wise logsumexp that waits for the pass that differentiates it: which kernels run, and that what it is worth does not
+depend on when it is read.
+
+Host logic only: CPU tensors stand in for device memory and plain torch for the kernels' entry points.
+"""
+
+import numpy as onp
+import pytest
+import torch
+
+from autograd_amd import core
+from autograd_amd._lib import Affine, Op, Red
+from autograd_amd.numpy import devarray as D
+from autograd_amd.numpy import fusion
+from autograd_amd.numpy.devarray import DevArray
+from autograd_amd.scipy.special import logsumexp
+
+ROWS, COLS = 100, 100
+
+
+def _value(operand):
+    if type(operand) is not Affine:
+        return operand
+    out = operand.t * operand.scale
+    out = out * operand.ascale if operand.ascale is not None else out
+    return out + operand.shift if operand.shift is not None else out
+
+
+def _write(x, S, ans, row_sums=None, col_factor=None, scaled=None, col_sums=None):
+    if row_sums is not None:
+        row_sums.copy_(S.sum(1, keepdim=True))
+    if scaled is not None:
+        scaled.copy_(S if col_factor is None else S * col_factor)
+    if col_sums is not None:
+        col_sums.copy_(((x.t if type(x) is Affine else x) * S).sum(0, keepdim=True))
+    return True
+
+
+@pytest.fixture
+def kernels(monkeypatch):
+    """Stand-ins for the launches; the list of entry points called, in order."""
+    calls = []
+
+    def lse_rows(code, x, g, ans=None, **wanted):
+        calls.append("rows" if ans is None else "rows+value")
+        lse = torch.logsumexp(_value(x), 1, keepdim=True)
+        if ans is not None:
+            ans.copy_(lse)
+        return _write(x, g * torch.exp(_value(x) - lse), lse, **wanted)
+
+    def lse_cotangent(code, x, ans, g, **wanted):
+        calls.append("tile")
+        return _write(x, g * torch.exp(_value(x) - ans), ans, **wanted)
+
+    def map_reduce(op, red, code, shape, mask, out, ins):
+        assert op == Op.COPY and red == Red.LOGSUMEXP
+        calls.append("reduce")
+        out.copy_(torch.logsumexp(_value(ins[0]), 1, keepdim=True))
+        return True
+
+    def elementwise(op, code, shape, outs, ins):
+        calls.append("copy" if op == Op.COPY else "rule" if op == Op.LSE_VJP else "other")
+        if op == Op.COPY:
+            outs[0].copy_(_value(ins[0]))
+        else:
+            assert op == Op.LSE_VJP
+            outs[0].copy_(_value(ins[0]) * _value(ins[1]) * torch.exp(_value(ins[2]) - _value(ins[3])))
+
+    monkeypatch.setattr(D._lib, "lse_rows", lse_rows)
+    monkeypatch.setattr(D._lib, "lse_cotangent", lse_cotangent)
+    monkeypatch.setattr(D._lib, "map_reduce", map_reduce)
+    monkeypatch.setattr(D._lib, "elementwise", elementwise)
+    monkeypatch.setattr(D._lib, "empty", lambda shape, dtype: torch.full(tuple(shape), float("nan"), dtype=D._lib.TORCH_DTYPE[dtype]))
+    monkeypatch.setattr(fusion, "ENABLED", False)
+    return calls
+
+
+def _matrix(fill, cols=COLS):
+    return DevArray(torch.full((ROWS, cols), float(fill), dtype=torch.float64))
+
+
+LSE = lambda A: logsumexp(A, axis=1)  # noqa: E731
+OF_ZEROS = onp.log(COLS)
+ONES = DevArray(torch.ones(ROWS, dtype=torch.float64))
+
+
+def test_a_logsumexp_that_has_run_is_not_formed_again(kernels):
+    A = _matrix(0.0)
+    vjp, val = core.make_vjp(LSE, A)
+    assert kernels == []
+    cotangent = vjp(ONES)
+    assert kernels == ["rows+value"]  # nobody read the value first: one pass forms both
+    vjp(ONES)
+    assert kernels == ["rows+value", "rule"]
+    del kernels[:]
+    vjp, val = core.make_vjp(LSE, A)
+    val._t
+    assert onp.array_equal(vjp(ONES)._t.numpy(), cotangent._t.numpy()) and kernels == ["reduce", "rule"]
+
+
+@pytest.mark.parametrize("cols,route", [(COLS, "tile"), (COLS + 1, "rows")])
+def test_the_consumers_of_a_cotangent_read_a_logsumexp_that_has_run(kernels, cols, route):
+    """Rows of whole vectors go to the kernel that reads the value; it does not take others, which go to the one pass."""
+    A, b = _matrix(0.0, cols), torch.linspace(0.5, 1.5, cols, dtype=torch.float64)
+
+    def wanted(ans):
+        S = D.LseCotangent(ONES._view(lambda t: t.reshape(ROWS, 1)), A, ans, A.dtype)
+        return [r._t for r in (S.scaled_by(b.expand(ROWS, cols)), S.row_sums(), S.col_sums_with(A))]
+
+    waiting = core.make_vjp(LSE, A)[1]
+    first = wanted(waiting)
+    assert kernels == ["rows+value"]
+    second = wanted(waiting)
+    assert kernels == ["rows+value", route]
+    assert all(torch.equal(x, y) for x, y in zip(first, second))
