@@ -18,8 +18,23 @@ from .builtins import tuple as atuple
 from .extend import defvjp_argnum, primitive, vspace
 from .wrap_util import unary_to_nary
 
-make_vjp = unary_to_nary(core.make_vjp)
+
+def _handed_over(value):
+    """A function's value as the caller receives it: deferred arithmetic is completed here, as the derivatives' is, so that
+    what the caller does to the inputs afterwards cannot reach it."""
+    settle = getattr(core, "settle", None)  # (a hosting package's core has none: values then stay as they are)
+    return settle(value) if settle is not None else value
+
+
+@unary_to_nary
+def make_vjp(fun, x):
+    """``(vjp, fun(x))`` where ``vjp(g)`` is the cotangent of the argument for the cotangent ``g`` of the value."""
+    pull_back, value = core.make_vjp(fun, x)
+    return pull_back, _handed_over(value)
+
+
 make_jvp = unary_to_nary(core.make_jvp)
+make_vjp_pending = unary_to_nary(core.make_vjp)  # for the package's own use: the value may still wait to be read
 
 
 def _anp(*values):
@@ -64,8 +79,7 @@ def grad(fun, x):
 def value_and_grad(fun, x):
     """Like ``grad``, returning ``(fun's value, gradient)`` from the one forward pass."""
     value, gradient = _seeded_with_ones(fun, x, "value_and_grad")
-    settle = getattr(core, "settle", None)  # (a hosting package's core has none: values then stay as they are)
-    return (settle(value) if settle is not None else value), gradient  # deferred arithmetic is completed here, as the gradient's is
+    return _handed_over(value), gradient
 
 
 @unary_to_nary
@@ -216,7 +230,8 @@ def grad_and_aux(fun, x):
     """For ``fun`` returning ``(value, aux)``: the gradient of ``value`` and ``aux`` as it is."""
     pull_back, (ans, aux) = core.make_vjp(lambda arg: atuple(fun(arg)), x)
     seed = (vspace(ans).ones(), vspace(aux).zeros())
-    return pull_back(seed), aux
+    gradient = pull_back(seed)
+    return gradient, _handed_over(aux)
 
 
 def multigrad_dict(fun):
@@ -253,5 +268,5 @@ def checkpoint(fun):
     """``fun`` as a primitive that keeps no intermediate values: its VJP traces ``fun`` again when
     the backward pass gets there (memory for recomputation)."""
     as_primitive = primitive(fun)
-    defvjp_argnum(as_primitive, lambda argnum, ans, args, kwargs: make_vjp(fun, argnum)(*args, **kwargs)[0])
+    defvjp_argnum(as_primitive, lambda argnum, ans, args, kwargs: make_vjp_pending(fun, argnum)(*args, **kwargs)[0])
     return as_primitive

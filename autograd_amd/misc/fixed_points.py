@@ -6,8 +6,8 @@ fixed point x* = f(a)(x*), the cotangent is  vjp_a( w )  where  w = g + J_x^T w 
 iteration (J_x is the Jacobian of f(a) at x*).  With device arrays, every step of both loops is kernel launches.
 """
 
-from .. import make_vjp
 from ..builtins import tuple as traced_tuple
+from ..differential_operators import make_vjp_pending
 from ..extend import defvjp, primitive, vspace
 
 
@@ -21,11 +21,11 @@ def fixed_point(f, a, x0, distance, tol):
 
 
 def _fixed_point_cotangent(ans, f, a, x0, distance, tol):
-    pull_back_a, _ = make_vjp(lambda p, x: f(p)(x))(a, ans)
+    pull_back_a, _ = make_vjp_pending(lambda p, x: f(p)(x))(a, ans)
 
     def iteration(packed):
         p, at, g = packed
-        pull_back_x, _ = make_vjp(f(p))(at)
+        pull_back_x, _ = make_vjp_pending(f(p))(at)
         space = vspace(at)
         return lambda w: space.add(pull_back_x(w), g)
 

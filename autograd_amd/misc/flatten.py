@@ -8,8 +8,8 @@ unflattening is slice + reshape views and launches nothing.
 """
 
 import autograd_amd.numpy as np
-from autograd_amd import make_vjp
 from autograd_amd.builtins import type
+from autograd_amd.differential_operators import make_vjp_pending
 
 
 def _leaves_in_order(value):
@@ -37,7 +37,7 @@ def flatten(value):
     """Flattens any nesting of tuples, lists, or dicts, with device arrays or scalars inside.
     Returns a 1-d device array and an unflatten function: unflattening a vector is the cotangent map
     of flattening, which hands every leaf its slice in the leaf's shape."""
-    unflatten, flat = make_vjp(_flatten)(value)
+    unflatten, flat = make_vjp_pending(_flatten)(value)
     return flat, unflatten
 
 

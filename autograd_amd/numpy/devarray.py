@@ -497,10 +497,11 @@ class LseCotangent(DevArray):
     Anything else reads ``_t`` as on any ``DevArray`` and gets the matrix written out.
     """
 
-    __slots__ = ("_g", "_x", "_ans", "_ans_kept", "_shape", "_wanted")
+    __slots__ = ("_g", "_x", "_ans", "_ans_kept", "_unwritten", "_shape", "_wanted")
 
-    def __init__(self, g_k, x, ans, dtype):
+    def __init__(self, g_k, x, ans, dtype, unwritten=True):
         self._g, self._x, self._ans = g_k, x, ans
+        self._unwritten = unwritten  # no array has been assigned into since `ans` was asked for: it is the logsumexp of `x` still
         self._ans_kept = None  # (rows, 1) form of `ans` once it has a value
         self._shape = x.shape
         self.dtype = dtype
@@ -520,9 +521,15 @@ class LseCotangent(DevArray):
         return out
 
     def _ans_waits(self):
-        """Whether the logsumexp itself has not run."""
+        """Whether the logsumexp itself has not run.  One that was asked of other memory than the array holds by now is run
+        here: the pass over what it holds now would not be its value."""
         ans = self._ans
-        return type(ans) is PendingReduce and ans._call is not None
+        if type(ans) is not PendingReduce or ans._call is None:
+            return False
+        if ans._call[3][0]._h().data_ptr() == self._x._h().data_ptr():
+            return True
+        ans._t
+        return False
 
     def _ans_tensor(self):
         kept = self._ans_kept
@@ -623,7 +630,7 @@ class LseCotangent(DevArray):
         outs = dict(row_sums=rs[1] if rs else None, col_factor=sc[0] if sc else None, scaled=sc[1] if sc else None,
                     col_sums=cs[1] if cs else None)
         waits = self._ans_waits()
-        if (waits and self._one_pass(**outs)) or self._from_ans(**outs) or (not waits and self._one_pass(**outs)):
+        if (waits and self._one_pass(**outs)) or self._from_ans(**outs) or (not waits and self._unwritten and self._one_pass(**outs)):
             return
         # a layout the fused kernel does not take after all: write the matrix out, then the plain kernels
         full = DevArray(self._t, self.dtype)
@@ -1262,12 +1269,39 @@ def reduce_shape(shape, axes, keepdims):
 _IDENTITY = {Red.SUM: 0.0, Red.PROD: 1.0}
 
 
+# reductions of arrays in memory that were left pending without marking the arrays (weakly held); an item assignment runs
+# those that are still waiting
+_WAITING = []
+_waiting_limit = 64
+
+
+def until_written(reduction):
+    """``reduction``, which keeps unmarked operands (``_kept``), noted to run before anything is assigned into an array."""
+    global _waiting_limit
+    if len(_WAITING) >= _waiting_limit:
+        _WAITING[:] = [ref for ref in _WAITING if (held := ref()) is not None and held._call is not None]
+        _waiting_limit = max(64, 2 * len(_WAITING))
+    _WAITING.append(weakref.ref(reduction))
+    return reduction
+
+
+def run_waiting_reductions():
+    """Run them: memory is about to be written, and any of them may read it through another handle (a view taken earlier
+    shares the memory and cannot be seen from here)."""
+    waiting = _WAITING[:]
+    del _WAITING[:]
+    for ref in waiting:
+        reduction = ref()
+        if reduction is not None:
+            reduction._t
+
+
 class PendingReduce(DevArray):
     """A reduction of pending elementwise expressions, not yet run: the forward value of a traced ``sum`` is often
     never read (``grad`` keeps the cotangents only), and running it would force its operand expression into memory
     first.  Reading ``_t`` runs it."""
 
-    __slots__ = ("_call", "_shape")
+    __slots__ = ("_call", "_shape", "__weakref__")
 
     def __init__(self, call, shape, dtype):
         self._call, self._shape = call, shape
@@ -1327,12 +1361,14 @@ class PendingReduce(DevArray):
 _DEFERRED = _DEFERRED + (PendingReduce,)
 
 
-def _kept(x):
+def _kept(x, mark=True):
     """An operand as a deferred reduction keeps it: the array is marked as read by something pending (an item assignment
     then moves the ARRAY's handle to a buffer of its own) and the reduction holds a handle of its own on the memory as it
-    is now."""
+    is now.  Without ``mark`` the array stays as it is: an item assignment runs the reduction first (``until_written``) and
+    writes in place, where views of the array see it."""
     if isinstance(x, DevArray):
-        x._borrowed = True
+        if mark:
+            x._borrowed = True
         kind = type(x)
         if kind is DevArray:
             return DevArray(x._t, x.dtype)

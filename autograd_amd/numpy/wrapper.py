@@ -1092,6 +1092,8 @@ def assign_items(A, idx, value):
     if isbox(value) or isbox(idx):
         raise TypeError("a traced value cannot be assigned into an array: build the result with concatenate / where")
     D.ITEM_WRITES += 1
+    if D._WAITING:
+        D.run_waiting_reductions()
     if type(A) is D.LazyDevArray:
         if A._view_of_pending and (A._scale != 1.0 or A._shift is not None or A._ascale is not None) and builtins.any(A._raw.stride()):
             # `y = 1 - x; v = y[1:]; v[:] = 0`: in NumPy the write reaches y; here y's value does not exist in memory yet and

@@ -34,9 +34,9 @@ def logsumexp(x, axis=None, b=1.0, keepdims=False):
             return D.PendingReduce((Op.COPY, Red.LOGSUMEXP, dt, (D._kept(x),), axes, True, None), (x.shape[0], 1), dt)
         if axes == (1,) and x.dtype == dt and trace_stack.top >= 0 and _rows_in_one_pass(x, keepdims):
             # Rows of a matrix while a trace is open: the rule's own pass over x forms the value as well (LseCotangent),
-            # so it waits for that pass; anything that reads it first runs the reduction.
-            return D.PendingReduce((Op.COPY, Red.LOGSUMEXP, dt, (D._kept(x),), axes, keepdims, None),
-                                   (x.shape[0], 1) if keepdims else (x.shape[0],), dt)
+            # so it waits for that pass; anything that reads it or assigns into an array first runs the reduction.
+            return D.until_written(D.PendingReduce((Op.COPY, Red.LOGSUMEXP, dt, (D._kept(x, mark=False),), axes, keepdims, None),
+                                                   (x.shape[0], 1) if keepdims else (x.shape[0],), dt))
         return D.map_reduce(Op.COPY, Red.LOGSUMEXP, dt, (x,), axes, keepdims)
     # weighted form, the way scipy evaluates it: m = max(x), log(sum(b * exp(x - m))) + m, with weights of either
     # sign (a negative total gives NaN, as there).  Two passes over x: the maximum, then the weighted sum
@@ -76,6 +76,7 @@ def _keep(a, shape, axis, keepdims):
 
 def _make_grad_logsumexp(ans, x, axis=None, b=1.0, keepdims=False):
     shape, dtype = np.shape(x), np.result_type(x)
+    writes = D.ITEM_WRITES
 
     def vjp(g):
         if BatchMode.active:
@@ -91,7 +92,7 @@ def _make_grad_logsumexp(ans, x, axis=None, b=1.0, keepdims=False):
                     and _rows_in_one_pass(x, keepdims) and D.LseCotangent.eligible(g_k, x, ans, dt)):
                 # rows of a matrix: the cotangent stays unwritten until its consumers are known; the usual
                 # ones (row sums, a rescaled copy, column sums of a product) then come out of one pass
-                return D.LseCotangent(g_k, x, ans, dt)
+                return D.LseCotangent(g_k, x, ans, dt, writes == D.ITEM_WRITES)
             ans_k = _keep(ans, shape, axis, keepdims)
             return D.map_op(Op.LSE_VJP, dt, g_k, b, x, ans_k)
         g_repeated, _ = repeat_to_match_shape(g, shape, dtype, axis, keepdims)

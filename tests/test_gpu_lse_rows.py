@@ -130,3 +130,31 @@ def test_a_pending_logsumexp_is_formed_by_the_pass_that_differentiates_it():
     assert onp.allclose(dA.numpy(), 2 * lse * S * b, rtol=1e-12, atol=1e-12)
     untraced = logsumexp(A, axis=1)
     assert type(untraced).__name__ == "DevArray"
+
+
+def test_values_handed_to_the_caller_do_not_follow_later_writes():
+    import autograd_amd as ag
+    import autograd_amd.numpy as dnp
+    from autograd_amd.scipy.special import logsumexp
+
+    rs = onp.random.RandomState(5)
+    for cols in (100, 101):
+        a, b, g = rs.randn(100, cols), rs.randn(100, cols), rs.randn(100)
+        want = scipy.special.logsumexp(a, axis=1)
+        A = dnp.array(a)
+        V = A[:50]
+        vjp, val = ag.make_vjp(lambda A: logsumexp(A, axis=1))(A)
+        V[:] = dnp.array(b[:50])
+        A[50:] = dnp.array(b[50:])
+        cotangent = vjp(dnp.array(g)).numpy()
+        assert onp.allclose(val.numpy(), want, rtol=1e-13)
+        assert onp.allclose(cotangent, g[:, None] * onp.exp(b - want[:, None]), rtol=1e-12)
+        A = dnp.array(a)
+        gradient, aux = ag.grad_and_aux(lambda A: (dnp.sum(A * A), logsumexp(A, axis=1)))(A)
+        A._t.fill_(5.0)
+        assert onp.allclose(aux.numpy(), want, rtol=1e-13) and onp.allclose(gradient.numpy(), 2 * a, rtol=1e-13)
+        A = dnp.array(a)
+        C = A * 2.0
+        value, gradient = ag.value_and_grad(lambda A: dnp.sum(logsumexp(A, axis=1)))(A)
+        A[:] = 0.0
+        assert onp.allclose(C.numpy(), 2 * a) and onp.allclose(float(value), want.sum())

@@ -8,7 +8,7 @@ import numpy as onp
 import pytest
 import torch
 
-from autograd_amd import core
+from autograd_amd import core, make_vjp
 from autograd_amd._lib import Affine, Op, Red
 from autograd_amd.numpy import devarray as D
 from autograd_amd.numpy import fusion
@@ -113,3 +113,75 @@ def test_the_consumers_of_a_cotangent_read_a_logsumexp_that_has_run(kernels, col
     second = wanted(waiting)
     assert kernels == ["rows+value", route]
     assert all(torch.equal(x, y) for x, y in zip(first, second))
+
+
+@pytest.mark.parametrize("cols", [COLS, COLS + 1])
+def test_consumers_of_a_cotangent_whose_operand_was_written_read_the_value(kernels, monkeypatch, cols):
+    A = _matrix(0.0, cols)
+    vjp, val = core.make_vjp(LSE, A)
+    A[:] = _matrix(5.0, cols)
+    S = D.LseCotangent(ONES._view(lambda t: t.reshape(ROWS, 1)), A, val, A.dtype, False)
+    sums = S.row_sums()
+    if cols == COLS:
+        assert onp.allclose(sums._t.numpy(), cols * onp.exp(5.0 - onp.log(cols)), rtol=1e-12) and kernels[-1] == "tile"
+    else:
+        monkeypatch.setattr(D, "map_reduce_into", lambda op, out, xs, axes: out.copy_(xs[0]._t.sum(1, keepdim=True)))
+        assert onp.allclose(sums._t.numpy(), cols * onp.exp(5.0 - onp.log(cols)), rtol=1e-12) and kernels[-1] == "rule"
+
+
+@pytest.mark.parametrize("traced", [core.make_vjp, lambda f, A: make_vjp(f)(A)])
+@pytest.mark.parametrize("write", ["array", "view", "row"])
+@pytest.mark.parametrize("cols", [COLS, COLS + 1])
+def test_a_value_stays_what_it_was_when_the_operand_is_written(kernels, traced, write, cols):
+    A, B = _matrix(0.0, cols), _matrix(5.0, cols)
+    V = A[:50]
+    vjp, val = traced(LSE, A)
+    if write == "array":
+        A[:] = B
+    elif write == "view":
+        V[:] = B[:50]
+    else:
+        A[0] = B[0]
+    now, lse = A._t.clone(), onp.log(cols)
+    cotangent = vjp(ONES)
+    assert onp.allclose(val._t.numpy(), lse, rtol=1e-14)
+    # the rule g * exp(x - ans) of the array as it is now, as NumPy's arrays give it
+    assert onp.allclose(cotangent._t.numpy(), torch.exp(now - lse).numpy(), rtol=1e-12)
+    assert onp.array_equal(V._t.numpy(), A._t.numpy()[:50])  # an array and its views stay one memory
+
+
+def test_a_write_inside_the_traced_function_does_not_reach_an_earlier_value(kernels):
+    A, C = _matrix(0.0), _matrix(1.0)
+    V = C[:50]
+    seen = []
+
+    def f(A):
+        seen.append(logsumexp(C, axis=1))
+        V[:] = A._value[:50]
+        return logsumexp(A, axis=1)
+
+    make_vjp(f)(A)
+    assert onp.allclose(seen[0]._t.numpy(), 1.0 + onp.log(COLS), rtol=1e-14)
+
+
+def test_a_value_is_not_taken_from_memory_its_operand_moved_to(kernels):
+    A = _matrix(0.0)
+    vjp, val = core.make_vjp(LSE, A)
+    A._t = _matrix(5.0)._t
+    vjp(ONES)
+    assert onp.allclose(val._t.numpy(), OF_ZEROS, rtol=1e-14)
+
+
+def test_a_value_handed_over_is_in_memory(kernels):
+    A = _matrix(0.0)
+    _, val = make_vjp(LSE)(A)
+    A._t.fill_(5.0)
+    assert onp.allclose(val._t.numpy(), OF_ZEROS, rtol=1e-14)
+
+
+def test_finished_reductions_leave_the_list_of_waiting_ones(kernels):
+    A = _matrix(0.0)
+    for _ in range(300):
+        vjp, _ = core.make_vjp(LSE, A)
+        vjp(ONES)
+    assert len(D._WAITING) <= 128
