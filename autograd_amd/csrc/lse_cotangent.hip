@@ -380,6 +380,10 @@ static int launch_lse_cotangent(const agmi_lse_cotangent &c, void *workspace, si
 // and any element alignment takes the same path.  Measured at 8192 x 4096 with the finish: 16 waves, 8 to a row, 2 vectors 54 us; 4
 // to a row, 4 vectors 56; blocks of 8 or 4 waves 53-60 and 63; 16 waves to a row 68; streaming or plain accesses alike.  Vectors that run along the columns (the factor of the pending map, an offset, the
 // factor of the scaled copy) are staged in LDS once per block.
+//
+// Whether row sums are wanted is an argument of the template: what an infinite g does to them needs two more conditional stores,
+// and the kernel's time follows its branches and registers (all results, against a kernel that ignored such a g: 1.00 on the
+// average of 36 sizes and both precisions, 1.03 at 8192 x 4096 float32; the copy alone with those stores compiled in: 1.04-1.07).
 constexpr int kLseRowsMaxBlocks = 256;                // one block per CU: 16 waves of up to 128 VGPRs (8 of 256) fill it
 constexpr size_t kLseRowsMaxLds = 144 * 1024;         // of the CU's 160 KB, beside the static exchange slots
 
@@ -418,7 +422,7 @@ constexpr int kLseRowsLoadPolicy = 2, kLseRowsStorePolicy = 2;
 __device__ __forceinline__ float larger(float a, float b) { return __builtin_fmaxf(a, b); }
 __device__ __forceinline__ double larger(double a, double b) { return __builtin_fmax(a, b); }
 
-template <typename T, int NW, int WR, int J, bool COLS>
+template <typename T, int NW, int WR, int J, bool COLS, bool ROWS>
 __global__ __launch_bounds__(NW * 64) void lse_cotangent_tile_rows(const LseRowsParams p) {
     constexpr int V = 16 / sizeof(T), R = NW / WR, NT = WR * 64;
     // sixteen waves of eight vectors: neither the next row nor the exponentials fit beside the row and the column sums
@@ -550,6 +554,8 @@ __global__ __launch_bounds__(NW * 64) void lse_cotangent_tile_rows(const LseRows
             if (lane == 0) {
                 pair_m[slot][wave] = m;
                 pair_s[slot][wave] = sum;
+                // (the row's sum as it nearly always is; a wave that knows better after the barrier writes over it)
+                if (ROWS && wr == 0 && valid) static_cast<T *>(p.row_sums)[r] = g;
             }
             // (two sets of slots in turn: a wave writes a set again only after the barrier that follows every read of it)
             __syncthreads();
@@ -564,32 +570,49 @@ __global__ __launch_bounds__(NW * 64) void lse_cotangent_tile_rows(const LseRows
             for (int k = 1; k < WR; k <<= 1) total += __shfl_xor(total, k, 64);
             own = from_lane(weight, wr);
         }
-        const bool finite = total - total == T(0) && top - top == T(0);  // (the total is at least one then)
-        if (wr == 0 && valid && (p.ans != nullptr || p.row_sums != nullptr)) {
+        // (finite: the total is at least one then.  The same in every lane, and the compiler is told so: a branch it took for a
+        // divergent one would hide from it how many stores are in flight, and the next row's loads would wait for all of them)
+        const bool finite = total - total == T(0) && top - top == T(0);
+        const bool plain = finite && g - g == T(0);
+        if (wr == 0 && valid && (ROWS || p.ans != nullptr)) {
             // all -inf: -inf; a +inf present: +inf unless there is a NaN too
             const T ans = finite ? top + m_log(total) : (total == total ? top : total);
             if (lane == 0) {
                 if (p.ans != nullptr) static_cast<T *>(p.ans)[r * p.ans_rs] = ans;
                 // the exponentials over their own total add up to one; a row whose logsumexp is not finite holds an
                 // exp(inf - inf) or an exp(NaN)
-                if (p.row_sums != nullptr) static_cast<T *>(p.row_sums)[r] = finite ? g : T(__builtin_nan(""));
+                if (ROWS && (WR == 1 || !finite)) static_cast<T *>(p.row_sums)[r] = finite ? g : T(__builtin_nan(""));
             }
         }
         const T bad = total == total ? top : total;  // ans, where it is not finite
-        const T gf = m == -kInf ? T(0) : (g * own) / total;
         const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(
             static_cast<T *>(p.scaled) + r * p.scaled_rs, 0, (valid && p.scaled != nullptr) ? row_bytes : 0u, 0x00020000);
+        const T gf = (g * own) / total;
 #pragma unroll
         for (int j = 0; j < J; ++j) {
             const vec_t fv = *reinterpret_cast<const vec_t *>(held + p.factor_slot * p.lds_pitch + here + j * NT * V);
             vec_t s, o;
-            if (!kLong && finite) {  // the same for the whole row
+            if (!kLong && plain) {
 #pragma unroll
                 for (int v = 0; v < V; ++v) s[v] = e[j][v] * gf;
             } else {
                 const vec_t x = mapped(j);
+                if (kLong && plain) {
 #pragma unroll
-                for (int v = 0; v < V; ++v) s[v] = !kLong || !finite ? g * exp_of_nonpositive(x[v] - bad) : exp_of_nonpositive(x[v] - ms) * gf;
+                    for (int v = 0; v < V; ++v) s[v] = exp_of_nonpositive(x[v] - ms) * gf;
+                } else {
+                    // as the rule has it: a g that is not finite multiplies last, and is NaN times an exponential that vanishes
+                    // (or whose share of the total does), and the row's sum is NaN with it
+                    const T from = finite ? ms : bad, share = finite ? own / total : T(1);
+                    bool vanishes = false;
+#pragma unroll
+                    for (int v = 0; v < V; ++v) {
+                        s[v] = g * (exp_of_nonpositive(x[v] - from) * share);
+                        if (ROWS) vanishes |= s[v] != s[v] && (full || (j * NT + t) * V + v < cols);
+                    }
+                    if (ROWS && valid && __any(vanishes) && lane == 0)
+                        static_cast<T *>(p.row_sums)[r] = T(__builtin_nan(""));
+                }
             }
 #pragma unroll
             for (int v = 0; v < V; ++v) {
@@ -627,18 +650,23 @@ __global__ __launch_bounds__(NW * 64) void lse_cotangent_tile_rows(const LseRows
     }
 }
 
-template <typename T, int NW, int WR, int J>
-static int launch_lse_rows_kernel(const LseRowsParams &p, bool cols, int blocks, size_t lds, hipStream_t s) {
-    const void *kernel = cols ? reinterpret_cast<const void *>(lse_cotangent_tile_rows<T, NW, WR, J, true>)
-                              : reinterpret_cast<const void *>(lse_cotangent_tile_rows<T, NW, WR, J, false>);
+template <typename T, int NW, int WR, int J, bool COLS, bool ROWS>
+static int launch_lse_rows_kernel(const LseRowsParams &p, int blocks, size_t lds, hipStream_t s) {
     if (lds > 64 * 1024) {  // has to be asked for
-        if (int rc = hip_check(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)),
+        if (int rc = hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(lse_cotangent_tile_rows<T, NW, WR, J, COLS, ROWS>),
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)),
                                "lse_rows LDS size"))
             return rc;
     }
-    if (cols) hipLaunchKernelGGL((lse_cotangent_tile_rows<T, NW, WR, J, true>), dim3(blocks), dim3(NW * 64), lds, s, p);
-    else hipLaunchKernelGGL((lse_cotangent_tile_rows<T, NW, WR, J, false>), dim3(blocks), dim3(NW * 64), lds, s, p);
+    hipLaunchKernelGGL((lse_cotangent_tile_rows<T, NW, WR, J, COLS, ROWS>), dim3(blocks), dim3(NW * 64), lds, s, p);
     return hip_check(hipGetLastError(), "lse_rows launch");
+}
+
+template <typename T, int NW, int WR, int J>
+static int launch_lse_rows_kernel(const LseRowsParams &p, bool cols, int blocks, size_t lds, hipStream_t s) {
+    if (p.row_sums != nullptr)
+        return cols ? launch_lse_rows_kernel<T, NW, WR, J, true, true>(p, blocks, lds, s) : launch_lse_rows_kernel<T, NW, WR, J, false, true>(p, blocks, lds, s);
+    return cols ? launch_lse_rows_kernel<T, NW, WR, J, true, false>(p, blocks, lds, s) : launch_lse_rows_kernel<T, NW, WR, J, false, false>(p, blocks, lds, s);
 }
 
 template <typename T>

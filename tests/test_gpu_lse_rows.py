@@ -76,31 +76,42 @@ def test_every_result_at_the_edges_of_the_variants(dtype, vectors, extra, rows):
 @pytest.mark.parametrize("dtype", [F32, F64])
 @pytest.mark.parametrize("cols", [7, 600, 5000, 16001])
 def test_rows_with_infinities_and_nans(dtype, cols):
-    """Special values travel as through the two separate kernels (scipy's logsumexp, then g * exp(x - ans))."""
+    """Special values, in the rows and in their cotangents, travel as through the two separate kernels (scipy's logsumexp, then
+    g * exp(x - ans)): an infinite g times an exponential that vanishes is NaN, in the matrix and in the row's sum, wherever
+    in the row it lies."""
     import torch
 
     from autograd_amd import _lib
 
     rs = onp.random.RandomState(cols)
     dev, code = _lib.device(), _lib.DTYPE_CODE[onp.dtype(dtype)]
-    x = rs.randn(12, cols).astype(dtype)
+    x = rs.randn(20, cols).astype(dtype)
     x[1], x[2, 3], x[3, 0], x[4, cols - 1], x[5] = -onp.inf, onp.inf, onp.nan, -onp.inf, onp.nan
     x[6, 1], x[6, 2] = onp.inf, onp.nan
     x[7] = -onp.inf
     x[7, cols // 2] = -1000.0
     x[8, :] = 80.0
     x[9, : cols // 2] = -onp.inf
-    t_x, t_g = torch.from_numpy(x).to(dev), torch.full((12, 1), 2.0, dtype=torch.float32 if dtype is F32 else torch.float64, device=dev)
+    g = onp.full((20, 1), 2.0, dtype)
+    g[11:20, 0] = onp.inf, onp.inf, -onp.inf, onp.nan, onp.inf, onp.nan, onp.inf, -onp.inf, onp.nan
+    x[12, cols - 1] = x[13, 0] = -1000.0  # (exp(x - ans) is 0 in both precisions)
+    x[14, : cols // 2] = x[15, : cols // 2] = -onp.inf
+    x[17], x[18, 1], x[19, 2] = -onp.inf, onp.inf, onp.nan
+    t_x, t_g = torch.from_numpy(x).to(dev), torch.from_numpy(g).to(dev)
     t_ans, row_sums, out = torch.empty_like(t_g), torch.empty_like(t_g), torch.empty_like(t_x)
     assert _lib.lse_rows(code, t_x, t_g, ans=t_ans, row_sums=row_sums, scaled=out)
     with onp.errstate(all="ignore"):
         m = onp.max(x.astype(F64), axis=1, keepdims=True)
         safe = onp.where(onp.isfinite(m), m, 0.0)
         ans = onp.log(onp.sum(onp.exp(x.astype(F64) - safe), axis=1, keepdims=True)) + safe
-        S = 2.0 * onp.exp(x.astype(F64) - ans)
-    for have, ref in ((t_ans, ans), (out, S), (row_sums, S.sum(1, keepdims=True))):
+        S = g.astype(F64) * onp.exp(x.astype(F64) - ans)
+        sums = S.sum(1, keepdims=True)
+    alone = torch.empty_like(row_sums)
+    assert _lib.lse_rows(code, t_x, t_g, row_sums=alone) and onp.array_equal(alone.cpu().numpy(), row_sums.cpu().numpy(), equal_nan=True)
+    for have, ref in ((t_ans, ans), (out, S), (row_sums, sums)):
         have = have.cpu().numpy().astype(F64)
         assert onp.array_equal(onp.isnan(have), onp.isnan(ref)) and onp.array_equal(onp.isinf(have), onp.isinf(ref))
+        assert onp.array_equal(have[onp.isinf(ref)], ref[onp.isinf(ref)])
         fine = onp.isfinite(ref)
         # (80 and -1000 bring the error of |ans| ulps that rounding ans leaves in exp(x - ans))
         assert onp.all(onp.abs(have[fine] - ref[fine]) <= 2048 * onp.finfo(dtype).eps * onp.maximum(onp.abs(ref[fine]), 1e-30))
