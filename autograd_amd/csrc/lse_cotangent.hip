@@ -570,9 +570,7 @@ __global__ __launch_bounds__(NW * 64) void lse_cotangent_tile_rows(const LseRows
             for (int k = 1; k < WR; k <<= 1) total += __shfl_xor(total, k, 64);
             own = from_lane(weight, wr);
         }
-        // (finite: the total is at least one then.  The same in every lane, and the compiler is told so: a branch it took for a
-        // divergent one would hide from it how many stores are in flight, and the next row's loads would wait for all of them)
-        const bool finite = total - total == T(0) && top - top == T(0);
+        const bool finite = total - total == T(0) && top - top == T(0);  // (the total is at least one then)
         const bool plain = finite && g - g == T(0);
         if (wr == 0 && valid && (ROWS || p.ans != nullptr)) {
             // all -inf: -inf; a +inf present: +inf unless there is a NaN too
