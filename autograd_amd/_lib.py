@@ -728,7 +728,7 @@ def lse_cotangent(code, x, ans, g, row_sums=None, col_factor=None, scaled=None, 
     if rc:
         _check(rc, "agmi_lse_cotangent_fused")
     if ev is not None:
-        _end_lse(ev, probe, x, (ans, g), col_factor, row_sums, scaled, col_sums)
+        _end_lse(ev, ("lse_cotangent",), probe, x, (ans, g), col_factor, row_sums, scaled, col_sums)
     return True
 
 
@@ -748,12 +748,12 @@ def lse_rows(code, x, g, ans=None, row_sums=None, col_factor=None, scaled=None, 
     if rc:
         _check(rc, "agmi_lse_rows_fused")
     if ev is not None:
-        _end_lse(ev, probe, x, (g,), col_factor, ans, row_sums, scaled, col_sums)
+        _end_lse(ev, ("lse_rows",), probe, x, (g,), col_factor, ans, row_sums, scaled, col_sums)
     return True
 
 
-def _end_lse(ev, probe, x, ins, col_factor, *outs):
-    _TIMER.end(ev, ("lse_cotangent",), (tuple(t for t in outs if t is not None), (x,) + ins + ((col_factor,) if col_factor is not None else ())),
+def _end_lse(ev, key, probe, x, ins, col_factor, *outs):
+    _TIMER.end(ev, key, (tuple(t for t in outs if t is not None), (x,) + ins + ((col_factor,) if col_factor is not None else ())),
                probe=probe if probe is not None and probe >= 0 else None)
 
 

@@ -169,3 +169,25 @@ def test_values_handed_to_the_caller_do_not_follow_later_writes():
         value, gradient = ag.value_and_grad(lambda A: dnp.sum(logsumexp(A, axis=1)))(A)
         A[:] = 0.0
         assert onp.allclose(C.numpy(), 2 * a) and onp.allclose(float(value), want.sum())
+
+
+@pytest.mark.parametrize("of", ["sum", "sum of squares"])  # the one pass; the reduction and the pass that reads its value
+def test_a_kernel_is_timed_under_the_key_it_reports(of):
+    """What ``bench.py`` does: find a kernel in an unrestricted timing, then time launches with its key only."""
+    import autograd_amd as ag
+    import autograd_amd.numpy as dnp
+    from autograd_amd import _lib
+    from autograd_amd.scipy.special import logsumexp
+
+    rs = onp.random.RandomState(3)
+    A, B, C = (dnp.asarray(v) for v in (rs.randn(300, 1000), rs.uniform(0.5, 1.5, 1000), rs.randn(300)))
+    lse = lambda A, B, C: logsumexp(A * B[None, :] + C[:, None], axis=1)
+    f = ag.grad((lambda *a: dnp.sum(lse(*a))) if of == "sum" else (lambda *a: dnp.sum(lse(*a) ** 2)), (0, 1, 2))
+    with _lib.KernelTimer() as kt:
+        f(A, B, C)
+    seen = kt.summary()
+    assert any(name.startswith("lse_cotangent_tile") for name in seen)
+    for name, row in seen.items():
+        with _lib.KernelTimer(only={row["key"]}) as kt:
+            f(A, B, C)
+        assert kt.summary()[name]["launches"] == row["launches"], (name, row["key"])
