@@ -497,11 +497,11 @@ class LseCotangent(DevArray):
     Anything else reads ``_t`` as on any ``DevArray`` and gets the matrix written out.
     """
 
-    __slots__ = ("_g", "_x", "_ans", "_ans_kept", "_unwritten", "_shape", "_wanted")
+    __slots__ = ("_g", "_x", "_ans", "_ans_kept", "_again", "_shape", "_wanted")
 
-    def __init__(self, g_k, x, ans, dtype, unwritten=True):
+    def __init__(self, g_k, x, ans, dtype, again=True):
         self._g, self._x, self._ans = g_k, x, ans
-        self._unwritten = unwritten  # no array has been assigned into since `ans` was asked for: it is the logsumexp of `x` still
+        self._again = again  # whether a logsumexp that has run may be formed again by the one pass (with its roundings, and of `x` as it is now)
         self._ans_kept = None  # (rows, 1) form of `ans` once it has a value
         self._shape = x.shape
         self.dtype = dtype
@@ -578,10 +578,13 @@ class LseCotangent(DevArray):
         return True
 
     @staticmethod
-    def eligible(g_k, x, ans, dtype):
+    def eligible(g_k, x, ans, dtype, one_pass):
         """Whether the cotangent of the rows of ``x`` can stay unwritten: everything in one floating dtype, a layout the
-        fused kernels cover, a logsumexp that has run or is pending as a reduction."""
+        fused kernels cover, a logsumexp that has run or is pending as a reduction.  Without ``one_pass`` (the kernel that
+        forms the logsumexp itself is not meant for these rows) one that has run, of rows of whole vectors."""
         if x.dtype != dtype or type(g_k) is not DevArray or g_k.dtype != dtype or not LseCotangent.takes(x):
+            return False
+        if not one_pass and (type(ans) is not DevArray or x.shape[1] % (16 // dtype.itemsize)):
             return False
         rows = x.shape[0]
         return g_k.shape == (rows, 1) and type(ans) in (DevArray, PendingReduce) and ans.dtype == dtype and ans.shape in ((rows,), (rows, 1))
@@ -630,7 +633,7 @@ class LseCotangent(DevArray):
         outs = dict(row_sums=rs[1] if rs else None, col_factor=sc[0] if sc else None, scaled=sc[1] if sc else None,
                     col_sums=cs[1] if cs else None)
         waits = self._ans_waits()
-        if (waits and self._one_pass(**outs)) or self._from_ans(**outs) or (not waits and self._unwritten and self._one_pass(**outs)):
+        if (waits and self._one_pass(**outs)) or self._from_ans(**outs) or (not waits and self._again and self._one_pass(**outs)):
             return
         # a layout the fused kernel does not take after all: write the matrix out, then the plain kernels
         full = DevArray(self._t, self.dtype)

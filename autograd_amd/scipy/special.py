@@ -57,11 +57,11 @@ def logsumexp(x, axis=None, b=1.0, keepdims=False):
 
 
 def _rows_in_one_pass(x, keepdims):
-    """Whether the rows of ``x`` go to the kernels that form their logsumexp and its cotangent together.  Short rows with
+    """Whether the rows of ``x`` go to the kernel that forms their logsumexp and its cotangent together.  Short rows with
     the axis kept (a log-softmax) belong to the chains around them instead, which form the value themselves.  Below 8192
-    elements (launches, not bytes, are the cost there: 20 us against 25 replayed even at 300 x 250) the separate kernels
-    stay, so that small programs keep the bits of their rule-by-rule evaluation; the pass rescales each exponential
-    where the rule subtracts the logsumexp first."""
+    elements the reduction runs first and the cotangent reads it, which keeps the bits of a rule-by-rule evaluation (the one
+    pass rescales each exponential where the rule subtracts the logsumexp first).  A gradient of sum(logsumexp(A*b + c)) at
+    64 x 64 float32, replayed: 11.8 us with the pass that reads the value, 14.8 with the rule's separate kernels."""
     return x.size >= 8192 and D.LseCotangent.takes(x) and not (keepdims and fusion.rows_fit_a_wave(x.shape, x.dtype))
 
 
@@ -88,11 +88,12 @@ def _make_grad_logsumexp(ans, x, axis=None, b=1.0, keepdims=False):
         if _concrete(g, ans, x, b):
             g_k = _keep(D.asarray(g), shape, axis, keepdims)
             dt = D._float_dtype(D.result_dtype(g_k, x, ans))
-            if (type(b) is float and b == 1.0 and len(shape) == 2 and D.normalize_axes(axis, 2) == (1,)
-                    and _rows_in_one_pass(x, keepdims) and D.LseCotangent.eligible(g_k, x, ans, dt)):
-                # rows of a matrix: the cotangent stays unwritten until its consumers are known; the usual
-                # ones (row sums, a rescaled copy, column sums of a product) then come out of one pass
-                return D.LseCotangent(g_k, x, ans, dt, writes == D.ITEM_WRITES)
+            if type(b) is float and b == 1.0 and len(shape) == 2 and D.normalize_axes(axis, 2) == (1,):
+                one_pass = _rows_in_one_pass(x, keepdims)
+                if D.LseCotangent.eligible(g_k, x, ans, dt, one_pass):
+                    # rows of a matrix: the cotangent stays unwritten until its consumers are known; the usual
+                    # ones (row sums, a rescaled copy, column sums of a product) then come out of one pass
+                    return D.LseCotangent(g_k, x, ans, dt, one_pass and writes == D.ITEM_WRITES)
             ans_k = _keep(ans, shape, axis, keepdims)
             return D.map_op(Op.LSE_VJP, dt, g_k, b, x, ans_k)
         g_repeated, _ = repeat_to_match_shape(g, shape, dtype, axis, keepdims)

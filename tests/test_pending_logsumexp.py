@@ -13,6 +13,7 @@ from autograd_amd._lib import Affine, Op, Red
 from autograd_amd.numpy import devarray as D
 from autograd_amd.numpy import fusion
 from autograd_amd.numpy.devarray import DevArray
+from autograd_amd.scipy import special
 from autograd_amd.scipy.special import logsumexp
 
 ROWS, COLS = 100, 100
@@ -113,6 +114,27 @@ def test_the_consumers_of_a_cotangent_read_a_logsumexp_that_has_run(kernels, col
     second = wanted(waiting)
     assert kernels == ["rows+value", route]
     assert all(torch.equal(x, y) for x, y in zip(first, second))
+
+
+@pytest.mark.parametrize("rows,cols,deferred", [(16, 8, True), (7, 1000, True), (90, 90, True), (90, 91, False), (81, 101, False)])
+def test_small_matrices_keep_the_pass_that_reads_the_value(kernels, monkeypatch, rows, cols, deferred):
+    """Below 8192 elements the value runs first; the cotangent of rows of whole vectors still stays unwritten."""
+    A = DevArray(torch.randn(rows, cols, dtype=torch.float64))
+    g = DevArray(torch.ones(rows, dtype=torch.float64))
+    ans = core.make_vjp(LSE, A)[1]
+    assert kernels == ["reduce"] and type(ans) is DevArray
+    S = special._make_grad_logsumexp(ans, A, axis=1)(g)
+    if not deferred:
+        assert type(S) is DevArray
+        return
+    assert type(S) is D.LseCotangent
+    S.row_sums()._t
+    assert kernels == ["reduce", "tile"]
+    # a layout the kernel refuses: the plain kernels, never the one pass
+    monkeypatch.setattr(D._lib, "lse_cotangent", lambda *a, **k: False)
+    monkeypatch.setattr(D, "map_reduce_into", lambda op, out, xs, axes: out.copy_(xs[0]._t.sum(1, keepdim=True)))
+    special._make_grad_logsumexp(ans, A, axis=1)(g).row_sums()._t
+    assert kernels == ["reduce", "tile", "rule"]
 
 
 @pytest.mark.parametrize("cols", [COLS, COLS + 1])
