@@ -676,7 +676,7 @@ def map_reduce_static(op, red, code, shape, reduce_mask, out, ins):
 
 
 _lse_cot = AgmiLseCotangent()
-LSE_ROWS_MAX_VECTORS = 8192  # 16-byte vectors in the longest row that agmi_lse_rows_fused takes
+LSE_ROWS_MAX_VECTORS = 8192  # 16-byte vectors in the longest row that agmi_lse_rows_fused takes (whole vectors: half of that)
 
 
 def _fill_lse_cotangent(x, g, row_sums, col_factor, scaled, col_sums):

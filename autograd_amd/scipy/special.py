@@ -62,7 +62,7 @@ def _rows_in_one_pass(x, keepdims):
     elements the reduction runs first and the cotangent reads it, which keeps the bits of a rule-by-rule evaluation (the one
     pass rescales each exponential where the rule subtracts the logsumexp first).  A gradient of sum(logsumexp(A*b + c)) at
     64 x 64 float32, replayed: 11.8 us with the pass that reads the value, 14.8 with the rule's separate kernels."""
-    return x.size >= 8192 and D.LseCotangent.takes(x) and not (keepdims and fusion.rows_fit_a_wave(x.shape, x.dtype))
+    return x.size >= 8192 and D.LseCotangent.takes_unformed(x) and not (keepdims and fusion.rows_fit_a_wave(x.shape, x.dtype))
 
 
 def _keep(a, shape, axis, keepdims):

@@ -137,6 +137,17 @@ def test_small_matrices_keep_the_pass_that_reads_the_value(kernels, monkeypatch,
     assert kernels == ["reduce", "tile", "rule"]
 
 
+@pytest.mark.parametrize("cols,waits", [(8192, True), (8194, False), (8193, True), (16383, True), (16384, False), (16385, False)])
+def test_a_value_waits_only_for_a_kernel_that_takes_its_rows(kernels, cols, waits):
+    A = DevArray(torch.zeros(4, cols, dtype=torch.float64))
+    vjp, val = core.make_vjp(LSE, A)
+    assert kernels == ([] if waits else ["reduce"])
+    if not waits and cols % 2 == 0:
+        S = special._make_grad_logsumexp(val, A, axis=1)(DevArray(torch.ones(4, dtype=torch.float64)))
+        S.row_sums()._t
+        assert kernels == ["reduce", "tile"]
+
+
 @pytest.mark.parametrize("cols", [COLS, COLS + 1])
 def test_consumers_of_a_cotangent_whose_operand_was_written_read_the_value(kernels, monkeypatch, cols):
     A = _matrix(0.0, cols)
