@@ -492,8 +492,7 @@ class LseCotangent(DevArray):
     once and produces all of them, and this matrix itself never reaches memory.  Under ``grad`` the logsumexp's
     own value has usually not run either (``special.logsumexp`` leaves it pending while a trace is open): the same pass
     forms it (``agmi_lse_rows_fused``; rows too long for that kernel: the reduction, then ``agmi_lse_cotangent_fused``).  A
-    logsumexp that has run is read, not formed again (``agmi_lse_cotangent_fused``: 44 us against 50 at 8192 x 4096 float32;
-    it takes rows of whole 16-byte vectors, the others go to the one pass all the same).
+    logsumexp that has run is read where that is the faster way (``run``).
     Anything else reads ``_t`` as on any ``DevArray`` and gets the matrix written out.
     """
 
@@ -513,12 +512,27 @@ class LseCotangent(DevArray):
             raise AttributeError(name)
         if self._wanted:
             self.run()
-        # (a logsumexp that has run is what the rule kernel reads: the maximum and the sum are not formed again)
-        out = _lib.empty(self._shape, self.dtype) if self._ans_waits() else None
-        if out is None or not self._one_pass(scaled=out):
-            out = map_op(Op.LSE_VJP, self.dtype, self._g, 1.0, self._x, DevArray(self._ans_tensor(), self.dtype))._t
+        shape = self._shape
+        out = _lib.empty(shape, self.dtype)
+        if not (self._ans_waits() and self._matrix_in_one_pass() and self._one_pass(True, scaled=out)):
+            ans = self._ans_tensor().expand(shape)
+            _lib.elementwise(Op.LSE_VJP, _lib.DTYPE_CODE[self.dtype], shape, (out,), (self._g._t.expand(shape), 1.0, self._operand(), ans))
         self._t = out
         return out
+
+    def _operand(self):
+        x = self._x
+        return x._affine() if type(x) is LazyDevArray else x._t
+
+    def _matrix_in_one_pass(self):
+        """Whether the matrix alone, of a logsumexp that has not run, comes from the pass that forms both.  It mostly does (4096 x
+        512 float32: 5.8 us against 11.0 for the reduction and the rule); but a wave takes a row at a time, however short, and
+        a row of more than 4096 vectors keeps a whole CU busy: many rows of a few vectors (100000 x 32 float32: 34 against
+        14.4 us) and few very long ones (40 x 20001 float32: 17.2 against 14.6, 40 x 10001 float64: 22.3 against 15.6) are
+        better off with the two kernels.  (A logsumexp that has run is always read: the rule takes 42 us at 8192 x 4096 float32,
+        the pass that forms it again 48.)"""
+        rows, cols = self._shape
+        return not (rows >= 65536 and cols <= 80) and not (rows < 128 and cols > _lib.LSE_ROWS_MAX_VECTORS // 2 * (16 // self.dtype.itemsize))
 
     def _ans_waits(self):
         """Whether the logsumexp itself has not run.  One that was asked of other memory than the array holds by now is run
@@ -526,7 +540,8 @@ class LseCotangent(DevArray):
         ans = self._ans
         if type(ans) is not PendingReduce or ans._call is None:
             return False
-        if ans._call[3][0]._h().data_ptr() == self._x._h().data_ptr():
+        kept, now = ans._call[3][0]._h(), self._x._h()
+        if kept is now or kept.data_ptr() == now.data_ptr():
             return True
         ans._t
         return False
@@ -537,25 +552,20 @@ class LseCotangent(DevArray):
             kept = self._ans_kept = self._ans._t.reshape(self._shape[0], 1)
         return kept
 
-    def _one_pass(self, **wanted):
-        """Everything asked for, and the logsumexp where it has not run, in one pass over ``x``; False: nothing has run."""
-        x, ans = self._x, self._ans
-        pending = self._ans_waits()
-        value = _lib.empty((self._shape[0], 1), self.dtype) if pending else None
-        operand = x._affine() if type(x) is LazyDevArray else x._t
-        if not _lib.lse_rows(_lib.DTYPE_CODE[self.dtype], operand, self._g._t, ans=value, **wanted):
+    def _one_pass(self, waits, **wanted):
+        """Everything asked for, and the logsumexp where it ``waits``, in one pass over ``x``; False: nothing has run."""
+        value = _lib.empty((self._shape[0], 1), self.dtype) if waits else None
+        if not _lib.lse_rows(_lib.DTYPE_CODE[self.dtype], self._operand(), self._g._t, ans=value, **wanted):
             return False
-        if pending:
-            ans.computed_as(value)
+        if waits:
+            self._ans.computed_as(value)
         return True
 
     def _from_ans(self, **wanted):
         """Everything asked for in one pass over ``x`` that reads the logsumexp; False: a layout that kernel does not take."""
         if self._shape[1] % (16 // self.dtype.itemsize):
-            return False
-        x = self._x
-        operand = x._affine() if type(x) is LazyDevArray else x._t
-        return _lib.lse_cotangent(_lib.DTYPE_CODE[self.dtype], operand, self._ans_tensor(), self._g._t, **wanted)
+            return False  # (the kernel would refuse them too)
+        return _lib.lse_cotangent(_lib.DTYPE_CODE[self.dtype], self._operand(), self._ans_tensor(), self._g._t, **wanted)
 
     @staticmethod
     def takes(x):
@@ -588,11 +598,11 @@ class LseCotangent(DevArray):
     @staticmethod
     def eligible(g_k, x, ans, dtype, one_pass):
         """Whether the cotangent of the rows of ``x`` can stay unwritten: everything in one floating dtype, a layout the
-        fused kernels cover, a logsumexp that has run or is pending as a reduction.  Without ``one_pass`` (the kernel that
-        forms the logsumexp itself is not meant for these rows) one that has run, of rows of whole vectors."""
-        if x.dtype != dtype or type(g_k) is not DevArray or g_k.dtype != dtype or not LseCotangent.takes(x):
+        fused kernels cover, a logsumexp that has run or is pending as a reduction.  ``one_pass``: the kernel that forms the
+        logsumexp itself is meant for these rows (``takes_unformed`` has been asked); otherwise it has run, and rows are whole vectors."""
+        if x.dtype != dtype or type(g_k) is not DevArray or g_k.dtype != dtype:
             return False
-        if not one_pass and (type(ans) is not DevArray or x.shape[1] % (16 // dtype.itemsize)):
+        if not one_pass and (type(ans) is not DevArray or x.shape[1] % (16 // dtype.itemsize) or not LseCotangent.takes(x)):
             return False
         rows = x.shape[0]
         return g_k.shape == (rows, 1) and type(ans) in (DevArray, PendingReduce) and ans.dtype == dtype and ans.shape in ((rows,), (rows, 1))
@@ -640,8 +650,13 @@ class LseCotangent(DevArray):
         cs = wanted.get("col_sums")
         outs = dict(row_sums=rs[1] if rs else None, col_factor=sc[0] if sc else None, scaled=sc[1] if sc else None,
                     col_sums=cs[1] if cs else None)
+        # A value that waits is formed by the one pass.  One that has run is read where that is the faster kernel or the only one
+        # that may run: its tiles are 256 vectors wide, so rows of up to 128 vectors leave half of it idle (sum(logsumexp**2),
+        # replayed, reading / forming again: 16384 x 64 float32 27.3 / 19.8 us, 4096 x 512 20.5 / 19.3, 16384 x 512 float64 77 / 82,
+        # 8192 x 4096 float32 76 / 80, float64 161 / 204).
         waits = self._ans_waits()
-        if (waits and self._one_pass(**outs)) or self._from_ans(**outs) or (not waits and self._again and self._one_pass(**outs)):
+        first = waits or (self._again and self._shape[1] <= 128 * (16 // self.dtype.itemsize))
+        if (first and self._one_pass(waits, **outs)) or self._from_ans(**outs) or (not first and self._again and self._one_pass(False, **outs)):
             return
         # a layout the fused kernel does not take after all: write the matrix out, then the plain kernels
         full = DevArray(self._t, self.dtype)
@@ -1312,10 +1327,11 @@ class PendingReduce(DevArray):
     never read (``grad`` keeps the cotangents only), and running it would force its operand expression into memory
     first.  Reading ``_t`` runs it."""
 
-    __slots__ = ("_call", "_shape", "__weakref__")
+    __slots__ = ("_call", "_shape", "for_one_pass", "__weakref__")
 
     def __init__(self, call, shape, dtype):
         self._call, self._shape = call, shape
+        self.for_one_pass = False  # a row-wise logsumexp left to the pass that differentiates it (`LseCotangent`)
         self.dtype = dtype
         self._borrowed = False
         self._shape_tuple = shape

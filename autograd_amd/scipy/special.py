@@ -35,8 +35,10 @@ def logsumexp(x, axis=None, b=1.0, keepdims=False):
         if axes == (1,) and x.dtype == dt and trace_stack.top >= 0 and _rows_in_one_pass(x, keepdims):
             # Rows of a matrix while a trace is open: the rule's own pass over x forms the value as well (LseCotangent),
             # so it waits for that pass; anything that reads it or assigns into an array first runs the reduction.
-            return D.until_written(D.PendingReduce((Op.COPY, Red.LOGSUMEXP, dt, (D._kept(x, mark=False),), axes, keepdims, None),
-                                                   (x.shape[0], 1) if keepdims else (x.shape[0],), dt))
+            value = D.PendingReduce((Op.COPY, Red.LOGSUMEXP, dt, (D._kept(x, mark=False),), axes, keepdims, None),
+                                    (x.shape[0], 1) if keepdims else (x.shape[0],), dt)
+            value.for_one_pass = True
+            return D.until_written(value)
         return D.map_reduce(Op.COPY, Red.LOGSUMEXP, dt, (x,), axes, keepdims)
     # weighted form, the way scipy evaluates it: m = max(x), log(sum(b * exp(x - m))) + m, with weights of either
     # sign (a negative total gives NaN, as there).  Two passes over x: the maximum, then the weighted sum
@@ -89,7 +91,8 @@ def _make_grad_logsumexp(ans, x, axis=None, b=1.0, keepdims=False):
             g_k = _keep(D.asarray(g), shape, axis, keepdims)
             dt = D._float_dtype(D.result_dtype(g_k, x, ans))
             if type(b) is float and b == 1.0 and len(shape) == 2 and D.normalize_axes(axis, 2) == (1,):
-                one_pass = _rows_in_one_pass(x, keepdims)
+                # (a value that was left waiting for the one pass was asked about then)
+                one_pass = _rows_in_one_pass(x, keepdims) if type(ans) is not D.PendingReduce else ans.for_one_pass
                 if D.LseCotangent.eligible(g_k, x, ans, dt, one_pass):
                     # rows of a matrix: the cotangent stays unwritten until its consumers are known; the usual
                     # ones (row sums, a rescaled copy, column sums of a product) then come out of one pass

@@ -99,9 +99,10 @@ def test_a_logsumexp_that_has_run_is_not_formed_again(kernels):
     assert onp.array_equal(vjp(ONES)._t.numpy(), cotangent._t.numpy()) and kernels == ["reduce", "rule"]
 
 
-@pytest.mark.parametrize("cols,route", [(COLS, "tile"), (COLS + 1, "rows")])
+@pytest.mark.parametrize("cols,route", [(256, "rows"), (258, "tile"), (257, "rows"), (259, "rows"), (8192, "tile"), (8194, "tile")])
 def test_the_consumers_of_a_cotangent_read_a_logsumexp_that_has_run(kernels, cols, route):
-    """Rows of whole vectors go to the kernel that reads the value; it does not take others, which go to the one pass."""
+    """Rows of more than 128 whole vectors go to the kernel that reads the value; it does not take others, and is slower for
+    shorter ones: those go to the one pass."""
     A, b = _matrix(0.0, cols), torch.linspace(0.5, 1.5, cols, dtype=torch.float64)
 
     def wanted(ans):
@@ -110,10 +111,21 @@ def test_the_consumers_of_a_cotangent_read_a_logsumexp_that_has_run(kernels, col
 
     waiting = core.make_vjp(LSE, A)[1]
     first = wanted(waiting)
-    assert kernels == ["rows+value"]
+    start = ["rows+value"] if cols <= 8192 else ["reduce", "tile"]
+    assert kernels == start
     second = wanted(waiting)
-    assert kernels == ["rows+value", route]
+    assert kernels == start + [route]
     assert all(torch.equal(x, y) for x, y in zip(first, second))
+
+
+@pytest.mark.parametrize("rows,cols,route", [(65536, 80, ["reduce", "rule"]), (65535, 80, ["rows+value"]), (65536, 81, ["rows+value"]),
+                                             (127, 8193, ["reduce", "rule"]), (128, 8193, ["rows+value"]), (127, 8192, ["rows+value"])])
+def test_a_matrix_comes_from_the_faster_of_the_two_ways(kernels, rows, cols, route):
+    A = DevArray(torch.zeros(rows, cols, dtype=torch.float64))
+    vjp, val = core.make_vjp(LSE, A)
+    out = vjp(DevArray(torch.ones(rows, dtype=torch.float64)))
+    assert kernels == route
+    assert onp.allclose(val._t.numpy(), onp.log(cols), rtol=1e-14) and onp.allclose(out._t[-1].numpy(), 1 / cols, rtol=1e-13)
 
 
 @pytest.mark.parametrize("rows,cols,deferred", [(16, 8, True), (7, 1000, True), (90, 90, True), (90, 91, False), (81, 101, False)])
@@ -155,7 +167,7 @@ def test_consumers_of_a_cotangent_whose_operand_was_written_read_the_value(kerne
     A[:] = _matrix(5.0, cols)
     S = D.LseCotangent(ONES._view(lambda t: t.reshape(ROWS, 1)), A, val, A.dtype, False)
     sums = S.row_sums()
-    if cols == COLS:
+    if cols == COLS:  # (never the one pass: it would form the logsumexp of what the array holds now)
         assert onp.allclose(sums._t.numpy(), cols * onp.exp(5.0 - onp.log(cols)), rtol=1e-12) and kernels[-1] == "tile"
     else:
         monkeypatch.setattr(D, "map_reduce_into", lambda op, out, xs, axes: out.copy_(xs[0]._t.sum(1, keepdim=True)))
