@@ -30,15 +30,16 @@ struct CorrParams {
     int64_t o_fs, o_ss, o_s[3];
     uint32_t p_total;    // P[0] * P[1] * P[2]
     uint32_t tiles;      // correlate_positions: blocks per filter-batch tile
-    // correlate_reduce: log2 of the lanes that share the innermost window axis and the contracted axis (the rest of the
-    // block shares the window's rows), threads in a block
-    int lane_bits, d_bits, threads;
     // correlate_tiled: a block covers 2^jt_bits images x 2^p1_bits rows x 2^p2_bits columns of output
     // (256 positions) and stages the H x W window of signal they read, per image, in LDS
     int jt_bits, p1_bits, p2_bits, H, W;
     int DT;                     // contracted indices staged per step
     uint32_t n_tj, n_t1, n_t2;  // tiles along each
     uint32_t s_elems_padded;    // LDS elements reserved for the signal tile (a multiple of 8)
+    // correlate_reduce: log2 of the lanes that share the innermost window axis and the contracted axis (the rest of the
+    // block shares the window's rows), threads in a block
+    int lane_bits, d_bits, threads;
+    int line;  // correlate_reduce: one convolved axis only (slot 2), which the threads walk as they otherwise walk the window's rows
 };
 
 constexpr int kTileLoads = 8;    // signal elements a thread stages per step: tiles of up to 2048 elements
@@ -293,20 +294,28 @@ __global__ __launch_bounds__(kReduceBlock) void correlate_reduce(const T *__rest
     for (int u = 0; u < PT; ++u) s_off[u] = (p2 + u < c.P[2] ? u : c.P[2] - 1 - p2) * c.s_s[2];
     // The window rows that meet the signal are found up front (the position is the same for the whole block),
     // so the inner loop is free of bounds tests and the loads of several rows are issued together.
-    T acc[TI][PT];
+    T acc[TI][PT], odd = T(0);  // (a single output's terms go to two sums in turn: half the chain)
 #pragma unroll
     for (int t = 0; t < TI; ++t)
 #pragma unroll
         for (int u = 0; u < PT; ++u) acc[t][u] = T(0);
-    const int64_t lo = b1 < 0 ? -b1 : 0;                                     // k1 in [lo, hi)
-    const int64_t hi = c.N[1] - b1 < c.K[1] ? c.N[1] - b1 : c.K[1];
-    const int64_t f_row = lanes_1 * c.f_s[1], s_row = lanes_1 * c.s_s[1];
+    // With a single convolved axis (K[0] = K[1] = 1) its taps are walked the same way: a loop over them with everything
+    // else inside ran one multiply-add per turn (100000 taps by 9, float32: 166 us with 256 threads).
+    const bool line = c.line;
+    const int ax = line ? 2 : 1;                                             // the axis walked
+    const int64_t bw = line ? b2 : b1;
+    const int64_t lo = bw < 0 ? -bw : 0;                                     // its taps: [lo, hi)
+    const int64_t hi = c.N[ax] - bw < c.K[ax] ? c.N[ax] - bw : c.K[ax];
+    const int walkers = line ? lanes_k : lanes_1, walker = line ? lk : l1;
+    const int64_t f_row = walkers * c.f_s[ax], s_row = walkers * c.s_s[ax];
+    const int64_t other = line ? b1 : b2;                                    // where the other of the two axes starts
+    const int64_t k_end = line ? (l1 == 0 ? 1 : 0) : c.K[2], n_other = c.N[3 - ax];
 #pragma unroll 1
-    for (int64_t k2 = lk; k2 < c.K[2]; k2 += lanes_k) {
-        const int64_t s2 = b2 + k2;
-        if (static_cast<uint64_t>(s2) >= static_cast<uint64_t>(c.N[2])) continue;
-        const T *f2 = filter + k2 * c.f_s[2] + (lo + l1) * c.f_s[1];
-        const T *sg2 = signal + j * c.s_bs + s2 * c.s_s[2] + (b1 + lo + l1) * c.s_s[1];
+    for (int64_t k2 = line ? 0 : lk; k2 < k_end; k2 += lanes_k) {
+        const int64_t s2 = other + k2;
+        if (static_cast<uint64_t>(s2) >= static_cast<uint64_t>(n_other)) continue;
+        const T *f2 = filter + k2 * c.f_s[3 - ax] + (lo + walker) * c.f_s[ax];
+        const T *sg2 = signal + j * c.s_bs + s2 * c.s_s[3 - ax] + (bw + lo + walker) * c.s_s[ax];
 #pragma unroll 1
         for (int64_t d = ld; d < c.D; d += lanes_d) {
 #pragma unroll 1
@@ -316,9 +325,9 @@ __global__ __launch_bounds__(kReduceBlock) void correlate_reduce(const T *__rest
                 const T *fr = f2 + d * c.f_ds + k0 * c.f_s[0];
                 const T *sr = sg2 + d * c.s_ds + s0 * c.s_s[0];
                 constexpr int U = TI * PT == 1 ? 4 : 1;  // rows in flight (more of them spill the 128 registers)
-                int64_t k1 = lo + l1;
+                int64_t k1 = lo + walker;
 #pragma unroll 1
-                for (; k1 + (U - 1) * lanes_1 < hi; k1 += U * lanes_1) {
+                for (; k1 + (U - 1) * walkers < hi; k1 += U * walkers) {
                     T fv[U][TI], sv[U][PT];
 #pragma unroll
                     for (int m = 0; m < U; ++m) {
@@ -332,13 +341,16 @@ __global__ __launch_bounds__(kReduceBlock) void correlate_reduce(const T *__rest
 #pragma unroll
                         for (int t = 0; t < TI; ++t)
 #pragma unroll
-                            for (int u = 0; u < PT; ++u) acc[t][u] = fused_mul_add(fv[m][t], sv[m][u], acc[t][u]);
+                            for (int u = 0; u < PT; ++u) {
+                                if (U > 1 && m % 2 != 0) odd = fused_mul_add(fv[m][t], sv[m][u], odd);
+                                else acc[t][u] = fused_mul_add(fv[m][t], sv[m][u], acc[t][u]);
+                            }
                     fr += U * f_row;
                     sr += U * s_row;
                 }
                 if constexpr (U == 1) continue;
 #pragma unroll 1
-                for (; k1 < hi; k1 += lanes_1) {
+                for (; k1 < hi; k1 += walkers) {
                     T fv[TI], sv[PT];
 #pragma unroll
                     for (int t = 0; t < TI; ++t) fv[t] = fr[f_off[t]];
@@ -361,7 +373,7 @@ __global__ __launch_bounds__(kReduceBlock) void correlate_reduce(const T *__rest
     for (int t = 0; t < TI; ++t)
 #pragma unroll
         for (int u = 0; u < PT; ++u) {
-            T v = acc[t][u];
+            T v = acc[t][u] + odd;
 #pragma unroll
             for (int half = 32; half > 0; half >>= 1) v = v + __shfl_down(v, half, 64);
             if (lane == 0) partial[wave][t * PT + u] = v;
@@ -414,8 +426,16 @@ void launch_reduce_tile(const agmi_correlation *a, const CorrParams &c, int64_t 
 
 // The tile of outputs per block: of the tiles that still give about one block per CU (192 of 256), the one with the fewest
 // loads in all.  Tiles along the innermost axis need every tap of it inside the signal.
+//
+// Threads in a block: 1024 where each of them still has 32 terms, 512 where it has sixteen, else 256 (a larger block costs its
+// launch and a longer combination: 150 outputs of 9216 terms, float32, take 5.5 us with 256, 5.0 with 512, 5.9 with 1024); and 256
+// where there are more blocks than CUs: one of 1024 threads fills a CU, and the last round is nearly empty (288 blocks of
+// 21120 terms, float32: 13.1 us with 1024 threads, 10.3 with 512, 9.0 with 256).
+// Lanes along the innermost window axis: the power of two that covers it, at most 256, and along the contracted axis likewise, at
+// most what is left.  Where it is the only axis, so many that a thread still has four of its taps to load at a time (but half a
+// wave, whose loads are neighbours), and what the contracted axis leaves.
 template <typename T>
-void launch_reduce(const agmi_correlation *a, const CorrParams &c, hipStream_t s) {
+void launch_reduce(const agmi_correlation *a, CorrParams &c, hipStream_t s) {
     const bool inside = c.pad[2] == 0 && c.P[2] + c.K[2] - 1 <= c.N[2];
     static const int tiles[][2] = {{1, 1}, {2, 1}, {4, 1}, {1, 3}, {2, 3}, {1, 5}, {2, 5}};
     int best = 0;
@@ -428,6 +448,15 @@ void launch_reduce(const agmi_correlation *a, const CorrParams &c, hipStream_t s
         best_blocks = blocks;
         best_loads = blocks * (ti + pt);
     }
+    const int64_t terms = c.D * c.K[0] * c.K[1] * c.K[2];
+    const int bits = best_blocks > 256 ? 8 : (terms >= 32 * 1024 ? 10 : (terms >= 16 * 512 ? 9 : 8));
+    c.threads = 1 << bits;
+    c.line = c.K[0] == 1 && c.K[1] == 1;
+    c.lane_bits = c.d_bits = 0;
+    const int64_t along = c.line ? std::min<int64_t>(c.K[2], std::max<int64_t>(ceil_div(c.K[2], 4), 32)) : std::min<int64_t>(c.K[2], 256);
+    while (c.lane_bits < bits && (int64_t(1) << c.lane_bits) < along) ++c.lane_bits;
+    while (c.lane_bits + c.d_bits < bits && (int64_t(1) << c.d_bits) < c.D) ++c.d_bits;
+    while (c.line && c.lane_bits + c.d_bits < bits && (int64_t(1) << c.lane_bits) < c.K[2]) ++c.lane_bits;
     switch (best) {
         case 0: launch_reduce_tile<T, 1, 1>(a, c, best_blocks, s); break;
         case 1: launch_reduce_tile<T, 2, 1>(a, c, best_blocks, s); break;
@@ -544,15 +573,20 @@ extern "C" int agmi_correlate(int dtype, const agmi_correlation *a, void *stream
     for (int cand : {2, 4, 8})
         if (c.I > cand / 2 && ceil_div(c.I, cand) * pairs >= 65536) tile = cand;
     if (tile == 1 && c.I * pairs < 16384 && r_total >= 64) tile = 0;
-    if (tile == 0) {
-        // blocks of 1024 once a thread of such a block still has four terms; lanes along the innermost window axis: the
-        // power of two that covers it, at most 256; along the contracted axis likewise, at most what is left
-        c.threads = r_total >= 4 * kReduceBlock ? kReduceBlock : kBlock;
-        const int bits = c.threads == kReduceBlock ? 10 : 8;
-        c.lane_bits = c.d_bits = 0;
-        while (c.lane_bits < 8 && (int64_t(1) << c.lane_bits) < c.K[2]) ++c.lane_bits;
-        while (c.lane_bits + c.d_bits < bits && (int64_t(1) << c.d_bits) < c.D) ++c.d_bits;
-    }
+    // (innermost axes of extent 1, the columns of an image convolved along its rows only, say, are dropped: the reduction's
+    // lanes lie along the innermost axis.  500 rows of one column, 9 taps, 128 images: 56 us with the lanes along the images)
+    if (tile == 0)
+        for (int d = 0; d < 2 && c.K[2] == 1 && c.N[2] == 1 && c.P[2] == 1 && c.pad[2] == 0; ++d)
+            for (int slot = 2; slot >= 0; --slot) {
+                const int from = slot - 1;
+                c.K[slot] = from >= 0 ? c.K[from] : 1;
+                c.N[slot] = from >= 0 ? c.N[from] : 1;
+                c.P[slot] = from >= 0 ? c.P[from] : 1;
+                c.pad[slot] = from >= 0 ? c.pad[from] : 0;
+                c.f_s[slot] = from >= 0 ? c.f_s[from] : 0;
+                c.s_s[slot] = from >= 0 ? c.s_s[from] : 0;
+                c.o_s[slot] = from >= 0 ? c.o_s[from] : 0;
+            }
     // The LDS-staged kernel when its tiles fit: 256 positions per block shaped to the output (columns
     // first), the window of signal they read within kTileLoads x 256 elements, the taps within
     // kFilterLoads x 256.

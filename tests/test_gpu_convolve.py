@@ -166,7 +166,12 @@ def test_pad_and_its_rules_are_exact(dtype):
 # (batch, channels in, channels out, image, window): one block per output with blocks of 256 and of 1024 threads, tiles of
 # outputs with remainders along the channels and the window (widths 1 ... 7), short and long contracted axes
 REDUCTIONS = [(3, 1, 1, (9, 9), (2, 2)), (40, 1, 6, (12, 12), (5, 5)), (33, 6, 16, (9, 10), (5, 5)), (64, 5, 13, (7, 9), (3, 3)),
-              (300, 2, 3, (5, 40), (1, 7)), (17, 8, 24, (6, 6), (4, 4)), (2, 7, 9, (40, 6), (5, 6)), (5, 3, 31, (11, 3), (3, 1))]
+              (300, 2, 3, (5, 40), (1, 7)), (17, 8, 24, (6, 6), (4, 4)), (2, 7, 9, (40, 6), (5, 6)), (5, 3, 31, (11, 3), (3, 1)),
+              # one convolved axis (walked across the block; 256, 512 and 1024 threads, lanes to spare), given as rows or as columns
+              (2, 1, 2, (1, 5000), (1, 9)), (3, 2, 3, (1, 1100), (1, 64)), (1, 1, 1, (1, 20000), (1, 5)), (128, 4, 4, (500, 1), (9, 1)),
+              (70, 1, 3, (130, 1), (2, 1)), (1, 2, 40, (1, 300), (1, 200)),
+              # more blocks than the machine holds at 1024 threads each
+              (64, 4, 8, (64, 3), (3, 3)), (3, 3, 16, (40, 40), (7, 7))]
 
 
 @pytest.mark.parametrize("dtype", ["float32", "float64"])
