@@ -380,9 +380,10 @@ __global__ __launch_bounds__(kBlock) void concat_kernel(const ConcatParams p, T 
     const I row = static_cast<I>(p.row), inner = static_cast<I>(p.inner);
     int lo = 0, hi = p.n_pieces - 1;  // the pieces this block can meet
     if (V > 1) {
+        // (worth its dependent scalar loads where a block is at most half a row)
         const I block_row = static_cast<I>(first) / row;
         const int64_t r_first = first - static_cast<int64_t>(block_row) * p.row;
-        if (r_first + kBlock * V <= p.row) {
+        if (p.row >= 2 * kBlock * V && r_first + kBlock * V <= p.row) {
             while (lo < hi && r_first >= p.end[lo]) ++lo;
             hi = lo;
             while (hi + 1 < p.n_pieces && r_first + kBlock * V > p.end[hi]) ++hi;
@@ -496,18 +497,25 @@ extern "C" int agmi_concat(int dtype, int64_t outer, int64_t inner, int n_pieces
         set_error("concat: dtype %d is not a floating type", dtype);
         return AGMI_ERR_ARG;
     }
-    // 16 bytes to a thread once that still gives two blocks per CU; below, a join is bound by the latency of one chain of
-    // loads, which a vector across a border between pieces lengthens (256 rows of 128 + 512 + 1 float32: 4 us with one
-    // element to a thread, and a recurrent net's gradient of 64 such steps took 2673 us with vectors of 16 bytes throughout).
+    // 16 bytes to a thread once that still gives two blocks per CU, four where few pieces make the walk cheap anyway, and where
+    // vectors rarely cross a border between pieces: one that does goes element by element, a walk for each, and its whole wave
+    // with it.  Measured, one element / 16 bytes to a thread, float32: 1000 rows of 32 pieces of 33 elements 13.2 / 26 us, 4096
+    // rows of 221 + 17 + 51 4.9 / 6.0, a million rows of 1 + 2 8.2 / 8.8; 4096 rows of 1000 + 1 10.3 / 7.5; 2000 rows of 8 pieces of 64,
+    // whose borders all lie between vectors, 5.5 / 4.2.  Below, a join is bound by the latency of one chain of loads, which
+    // a vector across a border lengthens (256 rows of 128 + 512 + 1 float32: 4 us with one element to a thread, and a
+    // recurrent net's gradient of 64 such steps took 2673 us with vectors of 16 bytes throughout).
     const int vec = dtype == AGMI_F32 ? 4 : 2;
-    const bool wide = p.n >= 512 * kBlock * vec;
+    bool aligned = true;
+    for (int k = 0; k < n_pieces; ++k) aligned &= p.end[k] % vec == 0;
+    const int64_t run = p.row / n_pieces;  // elements that a piece puts into a row, on the average
+    const bool wide = p.n >= (n_pieces >= 8 ? 512 : 1024) * kBlock * vec && (run >= 256 || (aligned && run >= 64));
     const int64_t blocks = ceil_div(p.n, kBlock * (wide ? vec : 1));
     if (blocks > 0x7fffffffLL) {
         set_error("concat: too many elements");
         return AGMI_ERR_UNSUPPORTED;
     }
     hipStream_t s = as_stream(stream);
-    set_kernel_name("concat_kernel");
+    set_kernel_name(wide ? "concat_kernel<16 bytes>" : "concat_kernel");
     if (dtype == AGMI_F32)
         wide ? launch_concat<float, 4>(p, blocks, s, out) : launch_concat<float, 1>(p, blocks, s, out);
     else
