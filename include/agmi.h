@@ -354,10 +354,13 @@ int agmi_lse_cotangent_fused(int dtype, const agmi_lse_cotangent *c, void *works
                              void *stream);
 
 /* The same results (and the logsumexp itself) in one pass over the operand, for a logsumexp that has not run: ans[r *
- * ans_stride] (may be NULL) is written, c->ans is not read.  Any number of columns up to 4096 vectors of 16 bytes (16384 float32,
- * 8192 float64) at any element alignment, and up to twice that where it is no whole number of vectors; col_factor NULL means a factor of one (`scaled` is then S itself).  Column sums
- * are staged per block (at most 256 rows of `cols` elements) in `workspace`; a smaller workspace means fewer blocks.
- * AGMI_ERR_UNSUPPORTED outside this. */
+ * ans_stride] (may be NULL) is written, c->ans is not read.  Any number of columns up to 4096 vectors of 16 bytes (16384
+ * float32, 8192 float64) at any element alignment, and up to twice that where it is no whole number of vectors; col_factor
+ * NULL means a factor of one (`scaled` is then S itself).  The array factor of the map, an offset along the columns and the
+ * factor of the copy (where it is another vector than the map's) are staged in LDS: with n of these beyond the first,
+ * n * ceil(row bytes / 16) * 16 plus the row padded to a power of two of 16-byte vectors (at least 64) must fit 144 KB (up to
+ * 2048 vectors always do).  Column sums are staged per block (at most 256 rows of `cols` elements) in `workspace`; a smaller
+ * workspace means fewer blocks.  AGMI_ERR_UNSUPPORTED outside this. */
 int agmi_lse_rows_fused(int dtype, const agmi_lse_cotangent *c, void *ans, int64_t ans_stride, void *workspace,
                         size_t workspace_bytes, void *stream);
 

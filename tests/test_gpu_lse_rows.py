@@ -22,6 +22,13 @@ def _tolerance(dtype, cols):
     return 64 * onp.finfo(dtype).eps
 
 
+def _fits(cols, dtype, staged):
+    """Whether ``staged`` column vectors beyond the first fit the LDS beside the padded row (as ``include/agmi.h`` states it)."""
+    vectors = -(-cols * onp.dtype(dtype).itemsize // 16)
+    padded = next(n for n in (64, 128, 256, 512, 1024, 2048, 4096, 8192) if vectors <= n)
+    return 16 * (staged * vectors + padded) <= 144 * 1024
+
+
 @pytest.mark.parametrize("dtype", [F32, F64])
 @pytest.mark.parametrize("vectors,extra,rows", EDGES)
 def test_every_result_at_the_edges_of_the_variants(dtype, vectors, extra, rows):
@@ -39,21 +46,23 @@ def test_every_result_at_the_edges_of_the_variants(dtype, vectors, extra, rows):
     t_mem = put(mem)[:, :cols]
     t_col, t_row, t_g = put(by_col), put(by_row), put(g)
     wide = lambda t: t.expand(rows, cols)
+    # operand, its value, column vectors staged beyond the first: with the copy's factor, without one, without the copy
     forms = {
-        "A*b + c": (_lib.Affine(t_mem, 1.0, wide(t_row), wide(t_col)), mem[:, :cols].astype(F64) * by_col + by_row),
-        "-A + b": (_lib.Affine(t_mem, -1.0, wide(t_col)), -mem[:, :cols].astype(F64) + by_col),
-        "A": (t_mem, mem[:, :cols].astype(F64)),
+        "A*b + c": (_lib.Affine(t_mem, 1.0, wide(t_row), wide(t_col)), mem[:, :cols].astype(F64) * by_col + by_row, (0, 1, 0)),
+        "-A + b": (_lib.Affine(t_mem, -1.0, wide(t_col)), -mem[:, :cols].astype(F64) + by_col, (2, 1, 1)),
+        "A": (t_mem, mem[:, :cols].astype(F64), (1, 0, 0)),
     }
     tol = _tolerance(dtype, cols)
-    for name, (operand, x) in forms.items():
+    for name, (operand, x, staged) in forms.items():
         ans = scipy.special.logsumexp(x, axis=1, keepdims=True)
         S = g.astype(F64) * onp.exp(x - ans)
         for factor in (t_col, None):
             kind = dict(dtype=t_mem.dtype, device=dev)
             out = torch.full((rows, pitch), 7.0, **kind)
             t_ans, row_sums, col_sums = torch.empty((rows, 1), **kind), torch.empty((rows, 1), **kind), torch.empty((1, cols), **kind)
-            if not _lib.lse_rows(code, operand, t_g, ans=t_ans, row_sums=row_sums, col_factor=factor, scaled=out[:, :cols], col_sums=col_sums):
-                assert vectors > 3000, name  # (two or three vectors along the longest rows do not fit the LDS)
+            taken = _lib.lse_rows(code, operand, t_g, ans=t_ans, row_sums=row_sums, col_factor=factor, scaled=out[:, :cols], col_sums=col_sums)
+            assert taken == _fits(cols, dtype, staged[factor is None]), name
+            if not taken:
                 continue
             want = S * by_col if factor is not None else S
             got = out.cpu().numpy()
@@ -67,10 +76,42 @@ def test_every_result_at_the_edges_of_the_variants(dtype, vectors, extra, rows):
             alone = torch.empty((rows, cols), **kind)
             assert _lib.lse_rows(code, operand, t_g, col_factor=factor, scaled=alone)
             assert onp.array_equal(alone.cpu().numpy(), got[:, :cols]), name
-            if not _lib.lse_rows(code, operand, t_g, col_sums=(again := torch.empty_like(col_sums))):
-                assert vectors > 3000, name
-                continue
-            assert torch.equal(again, col_sums), name
+            taken = _lib.lse_rows(code, operand, t_g, col_sums=(again := torch.empty_like(col_sums)))
+            assert taken == _fits(cols, dtype, staged[2]), name
+            assert not taken or torch.equal(again, col_sums), name
+
+
+@pytest.mark.parametrize("dtype", [F32, F64])
+@pytest.mark.parametrize("fits", [0, 1, 2.5, 40])  # rows of partial column sums that the workspace holds (none: one block)
+def test_a_smaller_workspace_is_met_with_fewer_blocks(dtype, fits):
+    import ctypes
+
+    import torch
+
+    from autograd_amd import _lib
+
+    rows, cols = 5003, 259
+    rs = onp.random.RandomState(11)
+    dev, code, size = _lib.device(), _lib.DTYPE_CODE[onp.dtype(dtype)], onp.dtype(dtype).itemsize
+    mem, g = rs.randn(rows, cols).astype(dtype), rs.uniform(0.5, 2.0, (rows, 1)).astype(dtype)
+    t_mem, t_g = torch.from_numpy(mem).to(dev), torch.from_numpy(g).to(dev)
+    t_ans, row_sums, scaled = torch.empty_like(t_g), torch.empty_like(t_g), torch.empty_like(t_mem)
+    col_sums = torch.empty((1, cols), dtype=t_mem.dtype, device=dev)
+    c = _lib._fill_lse_cotangent(t_mem, t_g, row_sums, None, scaled, col_sums)
+    held = int(fits * cols) * size
+    workspace = torch.full((held + 4096,), 7, dtype=torch.uint8, device=dev)
+    _lib.lib()
+    rc = _lib._LIB.agmi_lse_rows_fused(code, ctypes.byref(c), t_ans.data_ptr(), 1, workspace.data_ptr() if held else None, held, _lib._stream())
+    assert rc == 0
+    assert bool((workspace[held:] == 7).all())  # nothing is written past the workspace
+    x = mem.astype(F64)
+    ans = scipy.special.logsumexp(x, axis=1, keepdims=True)
+    S = g * onp.exp(x - ans)
+    tol = _tolerance(dtype, cols)
+    assert onp.all(onp.abs(t_ans.cpu().numpy() - ans) <= tol * onp.maximum(onp.abs(ans), 1))
+    assert onp.all(onp.abs(scaled.cpu().numpy() - S) <= tol * S) and onp.all(onp.abs(row_sums.cpu().numpy() - g) <= tol * g)
+    # (a block's rows are added one after the other: up to 5003 / 8 of them, and one round per block)
+    assert onp.all(onp.abs(col_sums.cpu().numpy() - (x * S).sum(0)) <= (tol + (rows / 8 + 256) * onp.finfo(dtype).eps) * onp.abs(x * S).sum(0))
 
 
 @pytest.mark.parametrize("dtype", [F32, F64])
