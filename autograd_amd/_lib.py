@@ -10,6 +10,7 @@ There is NO fallback: if the library is missing or a launch is rejected, the
 call raises.
 """
 
+import contextlib
 import ctypes
 import os
 import sys
@@ -269,6 +270,11 @@ def device():
 
 def _stream():
     return torch._C._cuda_getCurrentRawStream(_DEVICE.index)
+
+
+def on_stream(raw):
+    """Context in which launches go to the stream ``raw`` (what ``_stream()`` gave), current or not."""
+    return contextlib.nullcontext() if raw == _stream() else torch.cuda.stream(torch.cuda.ExternalStream(raw, device=_DEVICE))
 
 
 def empty(shape, np_dtype):

@@ -1295,8 +1295,8 @@ def reduce_shape(shape, axes, keepdims):
 _IDENTITY = {Red.SUM: 0.0, Red.PROD: 1.0}
 
 
-# reductions of arrays in memory that were left pending without marking the arrays (weakly held); an item assignment runs
-# those that are still waiting
+# reductions of arrays in memory that were left pending without marking the arrays (weakly held), each with the stream that was
+# current then; an item assignment runs those that are still waiting
 _WAITING = []
 _waiting_limit = 64
 
@@ -1305,21 +1305,23 @@ def until_written(reduction):
     """``reduction``, which keeps unmarked operands (``_kept``), noted to run before anything is assigned into an array."""
     global _waiting_limit
     if len(_WAITING) >= _waiting_limit:
-        _WAITING[:] = [ref for ref in _WAITING if (held := ref()) is not None and held._call is not None]
+        _WAITING[:] = [entry for entry in _WAITING if (held := entry[0]()) is not None and held._call is not None]
         _waiting_limit = max(64, 2 * len(_WAITING))
-    _WAITING.append(weakref.ref(reduction))
+    _WAITING.append((weakref.ref(reduction), _lib._stream()))
     return reduction
 
 
 def run_waiting_reductions():
     """Run them: memory is about to be written, and any of them may read it through another handle (a view taken earlier
-    shares the memory and cannot be seen from here)."""
+    shares the memory and cannot be seen from here).  Each on the stream it was asked for on: its operand is formed there, and
+    nothing has made the writer's stream wait for it."""
     waiting = _WAITING[:]
     del _WAITING[:]
-    for ref in waiting:
+    for ref, stream in waiting:
         reduction = ref()
-        if reduction is not None:
-            reduction._t
+        if reduction is not None and reduction._call is not None:
+            with _lib.on_stream(stream):
+                reduction._t
 
 
 class PendingReduce(DevArray):

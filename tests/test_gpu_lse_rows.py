@@ -232,3 +232,47 @@ def test_a_kernel_is_timed_under_the_key_it_reports(of):
         with _lib.KernelTimer(only={row["key"]}) as kt:
             f(A, B, C)
         assert kt.summary()[name]["launches"] == row["launches"], (name, row["key"])
+
+
+@pytest.mark.parametrize("asked_on_default", [False, True])
+def test_a_waiting_value_is_formed_on_the_stream_it_was_asked_for_on(asked_on_default):
+    import torch
+
+    import autograd_amd.numpy as dnp
+    from autograd_amd import core
+    from autograd_amd.scipy.special import logsumexp
+
+    a = onp.random.RandomState(7).randn(1024, 1024).astype(F32)
+    A, B = dnp.array(a), dnp.array(a)
+    side, default = torch.cuda.Stream(), torch.cuda.current_stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(default if asked_on_default else side):
+        X = A
+        for _ in range(50):  # the operand is a while in the making
+            X = dnp.dot(X, A) * F32(1 / 32)
+        X = dnp.settle(X)
+        _, val = core.make_vjp(lambda X: logsumexp(X, axis=1), X)
+    with torch.cuda.stream(side if asked_on_default else default):
+        B[0] = A[1]
+    torch.cuda.synchronize()
+    assert onp.allclose(val.numpy(), scipy.special.logsumexp(X.numpy().astype(F64), axis=1), rtol=1e-5)
+
+
+@pytest.mark.parametrize("cols", [1003, 8193, 12001])  # (the longer ones ask for more than 64 KB of LDS)
+def test_the_one_pass_is_recorded_and_replayed(cols):
+    import torch
+
+    import autograd_amd as ag
+    import autograd_amd.numpy as dnp
+    from autograd_amd.scipy.special import logsumexp
+
+    rs = onp.random.RandomState(cols)
+    f = ag.grad(lambda A, B, C: dnp.sum(logsumexp(A * B[None, :] + C[:, None], axis=1)), (0, 1, 2))
+    args = [dnp.array(v) for v in (rs.randn(40, cols), rs.uniform(0.5, 1.5, cols), rs.randn(40))]
+    replayed = ag.capture(f, *args)
+    for _ in range(3):
+        args = [dnp.array(v) for v in (rs.randn(40, cols), rs.uniform(0.5, 1.5, cols), rs.randn(40))]
+        got = [r.numpy() for r in replayed(*args)]
+        torch.cuda.synchronize()
+        for have, want in zip(got, f(*args)):
+            assert onp.array_equal(have, want.numpy())

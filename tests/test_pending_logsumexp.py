@@ -4,6 +4,8 @@ depend on when it is read.
 Host logic only: CPU tensors stand in for device memory and plain torch for the kernels' entry points.
 """
 
+import contextlib
+
 import numpy as onp
 import pytest
 import torch
@@ -37,10 +39,23 @@ def _write(x, S, ans, row_sums=None, col_factor=None, scaled=None, col_sums=None
     return True
 
 
+class _Calls(list):
+    """The entry points called, in order; ``streams``: those current at the reductions among them."""
+
+    def __init__(self):
+        self.stream, self.streams = 0, []
+
+    @contextlib.contextmanager
+    def on_stream(self, stream):
+        before, self.stream = self.stream, stream
+        yield
+        self.stream = before
+
+
 @pytest.fixture
 def kernels(monkeypatch):
     """Stand-ins for the launches; the list of entry points called, in order."""
-    calls = []
+    calls = _Calls()
 
     def lse_rows(code, x, g, ans=None, **wanted):
         calls.append("rows" if ans is None else "rows+value")
@@ -56,6 +71,7 @@ def kernels(monkeypatch):
     def map_reduce(op, red, code, shape, mask, out, ins):
         assert op == Op.COPY and red == Red.LOGSUMEXP
         calls.append("reduce")
+        calls.streams.append(calls.stream)
         out.copy_(torch.logsumexp(_value(ins[0]), 1, keepdim=True))
         return True
 
@@ -72,6 +88,8 @@ def kernels(monkeypatch):
     monkeypatch.setattr(D._lib, "map_reduce", map_reduce)
     monkeypatch.setattr(D._lib, "elementwise", elementwise)
     monkeypatch.setattr(D._lib, "empty", lambda shape, dtype: torch.full(tuple(shape), float("nan"), dtype=D._lib.TORCH_DTYPE[dtype]))
+    monkeypatch.setattr(D._lib, "_stream", lambda: calls.stream)
+    monkeypatch.setattr(D._lib, "on_stream", calls.on_stream)
     monkeypatch.setattr(fusion, "ENABLED", False)
     return calls
 
@@ -207,6 +225,17 @@ def test_a_write_inside_the_traced_function_does_not_reach_an_earlier_value(kern
 
     make_vjp(f)(A)
     assert onp.allclose(seen[0]._t.numpy(), 1.0 + onp.log(COLS), rtol=1e-14)
+
+
+def test_a_write_on_another_stream_runs_a_waiting_value_on_its_own(kernels):
+    """The value's operand is formed on the stream it was asked for on; the writer's stream has not waited for that."""
+    A, B = _matrix(0.0), _matrix(1.0)
+    kernels.stream = 7
+    _, val = core.make_vjp(LSE, A)
+    kernels.stream = 3
+    B[0] = A[0]
+    assert kernels == ["reduce", "copy"] and kernels.streams == [7] and kernels.stream == 3
+    assert onp.allclose(val._t.numpy(), OF_ZEROS, rtol=1e-14) and kernels == ["reduce", "copy"]
 
 
 def test_a_value_is_not_taken_from_memory_its_operand_moved_to(kernels):
