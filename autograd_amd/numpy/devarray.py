@@ -526,13 +526,12 @@ class LseCotangent(DevArray):
 
     def _matrix_in_one_pass(self):
         """Whether the matrix alone, of a logsumexp that has not run, comes from the pass that forms both.  It mostly does (4096 x
-        512 float32: 5.8 us against 11.0 for the reduction and the rule); but a wave takes a row at a time, however short, and
-        a row of more than 4096 vectors keeps a whole CU busy: many rows of a few vectors (100000 x 32 float32: 34 against
-        14.4 us) and few very long ones (40 x 20001 float32: 17.2 against 14.6, 40 x 10001 float64: 22.3 against 15.6) are
-        better off with the two kernels.  (A logsumexp that has run is always read: the rule takes 42 us at 8192 x 4096 float32,
-        the pass that forms it again 48.)"""
-        rows, cols = self._shape
-        return not (rows >= 65536 and cols <= 80) and not (rows < 128 and cols > _lib.LSE_ROWS_MAX_VECTORS // 2 * (16 // self.dtype.itemsize))
+        512 float32: 5.8 us against 11.0 for the reduction and the rule), but a wave takes a row at a time, however short: many
+        rows of a few vectors are better off with the two kernels (100000 x 32 float32: 34 against 14.4 us; 16384 x 64 8.5 against
+        8.4, and 23 against 36 eagerly).  (Few very long rows stay with the one pass for the host's sake: 40 x 20001 float32 17.2
+        against 14.6 us replayed, 23 against 37 eagerly.  A logsumexp that has run is always read: the rule takes 42 us at 8192 x
+        4096 float32, the pass that forms it again 48.)"""
+        return self._shape[0] < 65536 or self._shape[1] > 80
 
     def _ans_waits(self):
         """Whether the logsumexp itself has not run.  One that was asked of other memory than the array holds by now is run

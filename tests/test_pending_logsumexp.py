@@ -137,7 +137,7 @@ def test_the_consumers_of_a_cotangent_read_a_logsumexp_that_has_run(kernels, col
 
 
 @pytest.mark.parametrize("rows,cols,route", [(65536, 80, ["reduce", "rule"]), (65535, 80, ["rows+value"]), (65536, 81, ["rows+value"]),
-                                             (127, 8193, ["reduce", "rule"]), (128, 8193, ["rows+value"]), (127, 8192, ["rows+value"])])
+                                             (40, 8193, ["rows+value"])])
 def test_a_matrix_comes_from_the_faster_of_the_two_ways(kernels, rows, cols, route):
     A = DevArray(torch.zeros(rows, cols, dtype=torch.float64))
     vjp, val = core.make_vjp(LSE, A)
