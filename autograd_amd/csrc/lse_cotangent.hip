@@ -364,13 +364,14 @@ static int launch_lse_cotangent(const agmi_lse_cotangent &c, void *workspace, si
 // When the logsumexp itself has not run yet (its value is only wanted by the rules, as under `grad`), a row that
 // fits the registers of a few waves is read ONCE: its maximum and sum of exponentials give ans, and the very
 // exponentials, rescaled, are S.  Bound by HBM: mem read once, the scaled copy written once (the two-pass form reads mem
-// twice).  8192 x 4096 float32: 50 + 4 us (5.4 TB/s in the first kernel) against 75 us in three launches (26.6 + 44.2 + 4.0);
+// twice).  8192 x 4096 float32: 51.5 + 3.9 us (5.2 TB/s in the first kernel) against 75 us in three launches (26.6 + 44.0 + 4.1);
 // 3001 x 1999 float64, whose rows are no whole number of vectors: 33 us against 134 us in six launches.
 //
 // A block of 16 waves works on 16 / WR rows at a time, WR waves to a row, J vectors of 16 bytes per lane; one block per CU walks
 // the rows with a stride, so that column sums stay in registers from row to row and only 256 partial rows
-// reach memory.  The next rows' loads are issued before the current ones are worked on (64 KB in flight per CU at 4096
-// float32 columns; latency x bandwidth is about 50 KB).  Per row there is one exchange between waves and one barrier: each wave
+// reach memory.  The next rows' loads are issued before the current ones are worked on: 32 KB in flight per CU at 4096
+// float32 columns, where latency x bandwidth is about 50 KB (hence 5.2 TB/s and not the 6 of a copy; the registers hold no third
+// row beside the exponentials and the column sums).  Per row there is one exchange between waves and one barrier: each wave
 // takes the exponentials against its OWN maximum m_w and publishes (m_w, sum); after the barrier every wave combines
 // the WR pairs to (m, total) and S is its exponentials times g * exp(m_w - m) / total: one exponential per element, the
 // logarithm is only taken for the value of ans.
@@ -378,8 +379,9 @@ static int launch_lse_cotangent(const agmi_lse_cotangent &c, void *workspace, si
 // Rows are addressed through buffer descriptors of exactly one row: elements past its end load as zero (and are turned into
 // -inf, which neither maximum nor sum sees) and stores past it are dropped, dword by dword, so any number of columns
 // and any element alignment takes the same path.  Measured at 8192 x 4096 with the finish: 16 waves, 8 to a row, 2 vectors 54 us; 4
-// to a row, 4 vectors 56; blocks of 8 or 4 waves 53-60 and 63; 16 waves to a row 68; streaming or plain accesses alike.  Vectors that run along the columns (the factor of the pending map, an offset, the
-// factor of the scaled copy) are staged in LDS once per block.
+// to a row, 4 vectors 56; blocks of 8 or 4 waves 53-60 and 63; 16 waves to a row 68; streaming or plain accesses alike (these rows start
+// at 16-byte borders).  Vectors that run along the columns (the factor of the pending map, an offset, the factor of the
+// scaled copy) are staged in LDS once per block.
 //
 // Whether row sums are wanted is an argument of the template: what an infinite g does to them needs two more conditional stores,
 // and the kernel's time follows its branches and registers (all results, against a kernel that ignored such a g: 1.00 on the
